@@ -228,7 +228,8 @@ int launch_fast(const G4DecodeArgs& a, int t_alloc, size_t lds, hipStream_t st) 
 namespace g4 {
 namespace {
 
-// Whether the call takes the split-K path (bf16, head dims 128/256, rows longer than one split).
+// Whether the call takes the split-K path (bf16, head dims 128/256/512; automatically, rows longer than
+// the two-launch path's, over few pairs or where no one-launch kernel holds them).
 bool use_split_keys(const G4DecodeArgs& a) {
   if (a.dtype != G4_DTYPE_BF16 || (a.head_dim != 128 && a.head_dim != 256 && a.head_dim != 512)) return false;
   const int t_alloc = (a.capacity + 31) / 32 * 32;
@@ -262,22 +263,27 @@ int launch_split_keys(const G4DecodeArgs& a, hipStream_t st) {
   return G4_OK;
 }
 
-// Pairs from which the automatic choice takes the two-launch path for rows of at most 1024
-// slots: with fewer, one workgroup per CU holds a whole row and the one-launch kernels are faster
-// (measured: 128 pairs 19.3 vs 22.2 us, 512 pairs 71.8 vs 62.9 us on a 512-slot ring).
+// Where the automatic choice takes the two-launch path (us per call, D = 256, R = 4, HIP graph over 12
+// caches):
+// - rows of 513 .. 1024 slots: always (768 slots, three split-K launches before: 2 pairs 18.3 -> 10.7,
+//   64 pairs 22.5 -> 15.9, 128 pairs 30.6 -> 24.2, 192 pairs 42.6 -> 32.7), and every row at head dim
+//   512, which has no one-launch kernel;
+// - rows of at most 512 slots from 256 pairs (one launch 71.8, two 62.9 at 512 pairs). With fewer, one
+//   launch needs no workspace, and the automatic choice keeps to it; callers that hold a workspace
+//   can ask for two launches where those are faster (kernels.decode_attention does).
 constexpr int64_t kTwoPassMinPairs = 256;
+constexpr int64_t kTwoPassFewPairs = 32;  // up to here the scores launch spreads a row over more CUs
 
 bool two_pass_applies(const G4DecodeArgs& a) {
   return a.dtype == G4_DTYPE_BF16 && (a.head_dim == 128 || a.head_dim == 256 || a.head_dim == 512) &&
          a.capacity <= kTpMaxSlots;
 }
 
-// Head dim 512 (the reference's default global head dim) has no one-launch kernel: its rows take
-// the two-launch path up to 1024 slots and the split-K path beyond, whatever the pair count.
 bool use_two_pass(const G4DecodeArgs& a) {
   if (!two_pass_applies(a)) return false;
   if (a.num_splits == G4_DECODE_TWO_PASS || a.prep) return true;  // only this path fuses the preparation
-  return a.num_splits == 0 && (a.head_dim == 512 || (int64_t)a.batch * a.kv_heads >= kTwoPassMinPairs);
+  return a.num_splits == 0 && (a.head_dim == 512 || a.capacity > kSplitSlots ||
+                               (int64_t)a.batch * a.kv_heads >= kTwoPassMinPairs);
 }
 
 template <int D, int NCH>
@@ -286,19 +292,27 @@ void launch_tp_values(const G4DecodeArgs& a, const uint16_t* ws, int row_slots, 
                      dim3(tp_waves_v<NCH>() * 64), (size_t)a.group * tp_lds_stride(NCH) * 2, st, a, ws, row_slots);
 }
 
+template <int D, int NW>
+void launch_tp_scores(const G4DecodeArgs& a, uint16_t* ws, int row_slots, hipStream_t st) {
+  const int parts = ((a.capacity + 31) / 32 + NW - 1) / NW;
+  const dim3 grid((unsigned)((int64_t)a.batch * a.kv_heads * parts)), block(NW * 64);
+  if (a.prep)
+    hipLaunchKernelGGL((decode_bf16_tp_scores_kernel<D, true, NW>), grid, block, 0, st, a, ws, parts, row_slots, *a.prep);
+  else
+    hipLaunchKernelGGL((decode_bf16_tp_scores_kernel<D, false, NW>), grid, block, 0, st, a, ws, parts, row_slots,
+                       G4DecodePrep{});
+}
+
 template <int D>
 int launch_two_pass(const G4DecodeArgs& a, hipStream_t st) {
   const int64_t npairs = (int64_t)a.batch * a.kv_heads;
   const int cap_chunks = (a.capacity + 31) / 32;
-  const int parts = (cap_chunks + kTpWavesS - 1) / kTpWavesS;
   const int row_slots = twopass_row_slots(a.capacity);
   uint16_t* ws = reinterpret_cast<uint16_t*>(a.workspace);
-  if (a.prep)
-    hipLaunchKernelGGL((decode_bf16_tp_scores_kernel<D, true>), dim3((unsigned)(npairs * parts)), dim3(kTpWavesS * 64),
-                       0, st, a, ws, parts, row_slots, *a.prep);
+  if (npairs <= kTwoPassFewPairs)
+    launch_tp_scores<D, kTpWavesFew>(a, ws, row_slots, st);
   else
-    hipLaunchKernelGGL((decode_bf16_tp_scores_kernel<D, false>), dim3((unsigned)(npairs * parts)),
-                       dim3(kTpWavesS * 64), 0, st, a, ws, parts, row_slots, G4DecodePrep{});
+    launch_tp_scores<D, kTpWavesS>(a, ws, row_slots, st);
   if (cap_chunks <= 16)
     launch_tp_values<D, 16>(a, ws, row_slots, st);
   else if (cap_chunks <= 24)

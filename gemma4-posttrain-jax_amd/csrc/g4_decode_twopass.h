@@ -1,6 +1,6 @@
-// bf16 decode attention in two stream-ordered launches, for rows of at most 1024 slots over many
-// (b, kv head) pairs (the E2B rollout batch: the 512-slot sliding-window ring and the global
-// layers' linear cache); included by g4_decode.hip after g4_decode_splitk.h.
+// bf16 decode attention in two stream-ordered launches, for rows of at most 1024 slots (the 512-slot
+// sliding-window ring and the global layers' linear cache of a rollout; use_two_pass says where it
+// is the faster path); included by g4_decode.hip after g4_decode_splitk.h.
 //
 // The one-launch kernels keep a pair's whole row on one CU: K streams in, the row is scored, the
 // softmax runs behind barriers and the value pass follows, so every CU ends each pair with a
@@ -25,6 +25,10 @@
 // prepares the pair's q heads for itself, so 8 waves (two workgroups per 512-slot row) repeat it
 // half as often as 4 (E2B decode step 4.484 -> 4.473 ms; 16 waves, one workgroup per row: 4.561).
 constexpr int kTpWavesS = 8;
+// With so few pairs that the whole launch is one round trip to memory, 2 waves: a row's chunks spread
+// over four times the CUs (D = 256, 512 slots: 2 pairs 10.8 -> 9.3 us per call, 32 pairs 11.9 -> 10.6;
+// D = 512: 14.0 -> 11.0; at 64 pairs 8 waves are as fast).
+constexpr int kTpWavesFew = 2;
 // Waves per values workgroup. Every workgroup forms the exact probabilities of the pair's heads for
 // itself, so fewer, larger workgroups repeat less of that work: 8 waves (two workgroups per (b, kv
 // head) at D = 256) for rows of up to 16 chunks, where the kernel holds 102 VGPRs (E2B decode step
@@ -40,8 +44,8 @@ __host__ __device__ inline size_t twopass_workspace_bytes(int npairs, int R, int
   return (size_t)npairs * R * twopass_row_slots(capacity) * 2;
 }
 
-// grid: pairs x parts, parts = ceil(ceil(capacity / 32) / kTpWavesS); wave w of part p takes chunk
-// kTpWavesS * p + w.
+// grid: pairs x parts, parts = ceil(ceil(capacity / 32) / NW); wave w of part p takes chunk
+// NW * p + w.
 //
 // PREP: the launch also does g4_kv_append's work from the raw projection rows (G4DecodePrep). The
 // waves of a workgroup prepare the pair's R query heads once (prep_head: g4_kv_append's own
@@ -56,10 +60,11 @@ __host__ __device__ inline size_t twopass_workspace_bytes(int npairs, int R, int
 // LDS from q for the same reason (with the operand in registers, 138 registers and one workgroup
 // per CU: 30.1 us for a full 512-slot ring at B = 256; at head dim 512, 36 bytes of spills). Head
 // dim 512 holds 128 registers of K alone, so it takes no occupancy bound.
-template <int D, bool PREP>
-__global__ __launch_bounds__(kTpWavesS * 64, D <= 256 ? 4 : 1) void decode_bf16_tp_scores_kernel(G4DecodeArgs a, uint16_t* ws,
+template <int D, bool PREP, int NW>
+__global__ __launch_bounds__(NW * 64, D <= 256 ? 4 : 1) void decode_bf16_tp_scores_kernel(G4DecodeArgs a, uint16_t* ws,
                                                                               int parts, int row_slots,
                                                                               G4DecodePrep pp) {
+  static_assert(NW >= 2, "waves 0 and 1 prepare the new K and V rows");
   constexpr int PER = D / 64;
   constexpr bool kQlds = PREP || D >= 256;  // the q operand read from LDS
   __shared__ __attribute__((aligned(16))) uint16_t q_lds[kQlds ? 16 * D : 1];  // [R][D] (prepared) q
@@ -74,14 +79,14 @@ __global__ __launch_bounds__(kTpWavesS * 64, D <= 256 ? 4 : 1) void decode_bf16_
   KeyRange kr = key_range(a, b);
   if (PREP) kr.new_slot = pp.k_raw ? append_slot(a, kr.q) : -1;  // the append comes from the raw rows
   const int n_chunks = (kr.n_keys + 31) >> 5;
-  const int chunk = part * kTpWavesS + w;
+  const int chunk = part * NW + w;
   const int new_chunk = kr.new_slot >= 0 ? (int)(kr.new_slot >> 5) : -1;
   const bool writer = new_chunk == chunk;  // the wave that scores the appended slot's chunk
 
   // PREP: the preparation's loads go out first (they return before the K chunk: vector loads
   // complete in issue order), so its arithmetic runs while the K chunk is in flight
   const int h = pair - b * a.kv_heads;
-  const bool has_slot = PREP && pp.k_raw && new_chunk >= part * kTpWavesS && new_chunk < (part + 1) * kTpWavesS;
+  const bool has_slot = PREP && pp.k_raw && new_chunk >= part * NW && new_chunk < (part + 1) * NW;
   const bool kv_wave = has_slot && w < 2;  // wave 0: the new K row, wave 1: the new V row
   PrepIn<true, D> pq, pkv;
   const uint16_t* qrow = reinterpret_cast<const uint16_t*>(pp.q_raw) + (int64_t)b * pp.in_row_stride;
@@ -98,15 +103,15 @@ __global__ __launch_bounds__(kTpWavesS * 64, D <= 256 ? 4 : 1) void decode_bf16_
                                w == 0 ? reinterpret_cast<const uint16_t*>(pp.k_norm_weight) : nullptr,
                                w == 0 && (pp.flags & G4_APPEND_ROPE_K) != 0, rc, rs, lane);
   }
-  // without PREP from D = 256: thread t's 16-byte pieces t, t + 512 of the pair's q rows, requested
+  // without PREP from D = 256: thread t's 16-byte pieces t, t + 64 NW, ... of the pair's q rows, requested
   // ahead of the K chunk and stored to LDS once they land
-  constexpr int kQPieces = kQlds && !PREP ? (16 * D / 8 + kTpWavesS * 64 - 1) / (kTpWavesS * 64) : 1;
+  constexpr int kQPieces = kQlds && !PREP ? (16 * D / 8 + NW * 64 - 1) / (NW * 64) : 1;
   u32x4 qv[kQPieces];
   const int tid = threadIdx.x;
   if constexpr (kQlds && !PREP) {
 #pragma unroll
     for (int j = 0; j < kQPieces; ++j) {
-      const int t = tid + kTpWavesS * 64 * j;
+      const int t = tid + NW * 64 * j;
       qv[j] = t < R * D / 8 ? load16(reinterpret_cast<const uint16_t*>(a.q) + (int64_t)pair * R * D + 8 * t)
                             : u32x4{0u, 0u, 0u, 0u};
     }
@@ -146,7 +151,7 @@ __global__ __launch_bounds__(kTpWavesS * 64, D <= 256 ? 4 : 1) void decode_bf16_
                          (pp.flags & G4_APPEND_ROPE_Q) != 0, pp.eps);
       st_bf16<PER>(q_lds + w * D + lane * PER, pq.x);
     }
-    for (int r = w + kTpWavesS; r < R; r += kTpWavesS) {  // more than one head per wave (R > 4)
+    for (int r = w + NW; r < R; r += NW) {  // more than one head per wave (R > 4)
       float x[PER];
       prep_head<true, D, true>(qrow + (int64_t)(h * R + r) * D, reinterpret_cast<const uint16_t*>(pp.q_norm_weight),
                                (pp.flags & G4_APPEND_NORM_Q) != 0, (pp.flags & G4_APPEND_ROPE_Q) != 0, rc, rs, pp.eps,
@@ -169,7 +174,7 @@ __global__ __launch_bounds__(kTpWavesS * 64, D <= 256 ? 4 : 1) void decode_bf16_
   } else if constexpr (kQlds) {
 #pragma unroll
     for (int j = 0; j < kQPieces; ++j) {
-      const int t = tid + kTpWavesS * 64 * j;
+      const int t = tid + NW * 64 * j;
       if (t < R * D / 8) reinterpret_cast<u32x4*>(q_lds)[t] = qv[j];
     }
     wg_barrier();  // q rows in LDS

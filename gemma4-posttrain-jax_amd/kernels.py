@@ -147,6 +147,20 @@ def prepare_q(
     _lib.check(_lib.lib().g4_kv_append(ctypes.byref(a), _stream()), "g4_kv_append")
 
 
+def _decode_mode(num_splits: int, pairs: int, layer: LayerKVCache) -> int:
+    """``num_splits`` of a decode call: where the caller leaves the choice open, the two-launch path also
+    for bf16 rows of at most 512 slots at head dim 256 over so few (b, kv head) pairs that a row on two
+    CUs is the longer chain, or over more pairs than the one-launch kernel's two workgroups per pair
+    have CUs (us per call, one / two launches: 2 pairs 10.7 / 9.3, 32 pairs 11.5 / 10.6, 64 pairs
+    11.9 / 12.3, 128 pairs 15.9 / 17.1, 192 pairs 26.8 / 24.2; at head dim 128 one launch is as fast
+    or faster at every count). The library's own choice there is the path without a workspace."""
+
+    if (num_splits == 0 and layer.key.dtype == torch.bfloat16 and layer.head_dim == 256 and layer.capacity <= 512
+            and (pairs <= 32 or 128 < pairs < 256)):
+        return _lib.G4_DECODE_TWO_PASS
+    return num_splits
+
+
 def decode_attention(
     layer: LayerKVCache,
     q: torch.Tensor,
@@ -162,7 +176,7 @@ def decode_attention(
 ) -> torch.Tensor:
     """g4_decode_attention: q ``[B, Hkv, R, D]`` against ``layer``; returns ``[B, Hkv, R, D]``.
     With ``new_k``/``new_v`` (``[B, Hkv, D]``) the token's K/V is stored at ``q_pos`` first.
-    ``num_splits``: 0 lets the library choose; 1 or 2 workgroups per (b, kv head) in one pass;
+    ``num_splits``: 0 chooses automatically; 1 or 2 workgroups per (b, kv head) in one pass;
     ``_lib.G4_DECODE_SPLIT_KEYS`` splits the key range (long rows). A workspace of the size the
     library asks for is allocated from torch's caching allocator on the current stream; with
     ``no_alloc`` the call goes to g4_decode_attention_noalloc, which uses the library's own
@@ -194,7 +208,7 @@ def decode_attention(
         q_pos_scalar=qp_scalar, q_pos=qp_ptr, key_mask=_ptr(key_mask), key_mask_stride=key_mask.stride(0),
         q=_ptr(q), cache_k=_ptr(layer.key), cache_vt=_ptr(layer.value_t), cache_k_w=_ptr(layer.key),
         new_k=_ptr(new_k), new_v=_ptr(new_v), out=_ptr(out), workspace=None, workspace_bytes=0, prep=None,
-        num_splits=num_splits,
+        num_splits=_decode_mode(num_splits, B * H, layer),
     )
     if no_alloc:
         _lib.check(_lib.lib().g4_decode_attention_noalloc(ctypes.byref(a), _stream()), "g4_decode_attention_noalloc")
@@ -231,11 +245,13 @@ def decode_attention_fused(
     rope_cos / rope_sin f32 ``[B, D]``. Returns ``[B, Hkv, R, D]``."""
 
     B, H, R, D = q_raw.shape
-    stride = q_raw.stride(0)
-    if q_raw.dtype != layer.key.dtype or q_raw.stride(3) != 1 or q_raw.stride(2) != D or q_raw.stride(1) != R * D:
+    stride = q_raw.stride(0) if B > 1 else H * R * D  # one row: a view's batch stride is arbitrary
+    if q_raw.dtype != layer.key.dtype or q_raw.stride(3) != 1 or (R > 1 and q_raw.stride(2) != D) or (
+            H > 1 and q_raw.stride(1) != R * D):
         raise ValueError("q_raw must hold [Hkv, R, D] contiguous rows in the cache dtype")
     for name, t in (("k_raw", k_raw), ("v_raw", v_raw)):
-        if t is not None and (tuple(t.shape) != (B, H, D) or t.stride(0) != stride or t.stride(1) != D
+        if t is not None and (tuple(t.shape) != (B, H, D) or (B > 1 and t.stride(0) != stride)
+                              or (H > 1 and t.stride(1) != D)
                               or t.stride(2) != 1 or t.dtype != q_raw.dtype):
             raise ValueError(f"{name} must be [B, Hkv, D] rows sharing q_raw's batch stride")
     if (k_raw is None) != (v_raw is None):

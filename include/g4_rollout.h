@@ -187,15 +187,15 @@ typedef struct G4DecodeArgs {
 
 /* num_splits value: split-K over 512-slot key ranges in three launches (scores, values,
  * combine), for long rows over few (b, kv head) pairs. Uses the workspace. The automatic
- * choice takes it for bf16 rows longer than 512 slots when B * Hkv < 256 or when a one-pass
+ * choice takes it for bf16 rows longer than 1024 slots when B * Hkv < 256 or when a one-pass
  * row does not fit in LDS, and at head dim 512 for every row beyond the two-launch path's. */
 #define G4_DECODE_SPLIT_KEYS (-1)
 
 /* num_splits value: two stream-ordered launches for rows of at most 1024 slots (bf16, head dims
  * 128/256/512): the first scores K chunk by chunk into the workspace, the second forms the exact
  * probabilities and runs the value product, one wave per 16-row block of V^T. Uses the
- * workspace (bf16 scores [B * Hkv][R][512 or 1024]). The automatic choice takes it for such rows
- * when B * Hkv >= 256, and at head dim 512 always. */
+ * workspace (bf16 scores [B * Hkv][R][512 or 1024]). The automatic choice takes it for rows of
+ * more than 512 slots, when B * Hkv >= 256, and at head dim 512 always. */
 #define G4_DECODE_TWO_PASS (-2)
 
 /* Bytes of workspace the call described by args needs (0 when the chosen path uses none). The

@@ -1,0 +1,68 @@
+"""Small decode batches: the kernels and dispatch lines that only few rows reach, at the edges of their
+ranges (the larger batches are covered beside each kernel's own tests)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gemma4_posttrain_jax_amd import _lib, kernels
+from gemma4_posttrain_jax_amd.kvcache import new_layer_cache
+from gemma4_posttrain_jax_amd.model import rotary_tables
+from oracle import g4_oracle as O
+from test_gpu_kernels import _decode_case
+
+pytestmark = pytest.mark.gpu
+
+APPEND_FLAGS = (_lib.G4_APPEND_NORM_Q | _lib.G4_APPEND_ROPE_Q | _lib.G4_APPEND_NORM_K | _lib.G4_APPEND_ROPE_K
+                | _lib.G4_APPEND_NORM_V)
+
+
+# 32 / 34 pairs: the last count whose scores launch runs 2-wave workgroups and the first that does not;
+# 512 / 513 slots: the one-launch kernel's longest row and the first that only two launches take
+@pytest.mark.parametrize("B,D,ring,cap", [(1, 256, True, 512), (16, 256, True, 512), (17, 256, False, 512),
+                                          (1, 256, False, 513), (66, 256, True, 512), (16, 128, False, 700),
+                                          (17, 512, False, 33), (2, 512, False, 1024)])
+def test_decode_few_pairs_automatic(device, B, D, ring, cap):
+    rng = np.random.default_rng(B + D + cap)
+    q_pos = rng.integers(cap, 3 * cap, B) if ring else rng.integers(0, cap, B)
+    km = np.ones((B, max(cap, int(q_pos.max()) + 1)), bool)
+    km[0, : int(q_pos[0]) // 2] = False  # a left-padded row
+    _decode_case(device, O.BF16, B=B, H=2, R=4, D=D, cap=cap, ring=ring, window=cap if ring else 0, q_pos=q_pos,
+                 key_mask=km, fused=True, seed=cap + B)
+
+
+@pytest.mark.parametrize("R,ring,cap", [(4, True, 512), (1, False, 768), (16, True, 100)])
+def test_fused_preparation_of_one_row(device, R, ring, cap):
+    """One row (its batch stride is arbitrary) through the fused preparation: bit for bit the append and
+    the attention run separately."""
+
+    B, H, D = 1, 2, 256
+    g = torch.Generator(device="cuda").manual_seed(R + cap)
+    qkv = torch.randn((B, 1, (H * R + 2 * H) * D), device="cuda", generator=g).to(torch.bfloat16)
+    q = qkv[..., :H * R * D].view(B, 1, H, R, D)
+    k = qkv[..., H * R * D:(H * R + H) * D].view(B, 1, H, D)
+    v = qkv[..., (H * R + H) * D:].view(B, 1, H, D)
+    layers = [new_layer_cache(B, H, D, cap, ring, torch.bfloat16, device) for _ in range(2)]
+    layers[0].key.normal_(generator=g)
+    layers[0].value_t.normal_(generator=g)
+    layers[1].key.copy_(layers[0].key)
+    layers[1].value_t.copy_(layers[0].value_t)
+    pos = cap + 7 if ring else cap - 1
+    q_pos = torch.full((B,), pos, dtype=torch.int32, device=device)
+    km = torch.ones((B, pos + 1), dtype=torch.bool, device=device)
+    w = [(1 + 0.1 * torch.randn(D, device="cuda", generator=g)).to(torch.bfloat16) for _ in range(2)]
+    inv = (1.0 / (10000.0 ** (torch.arange(0, D, 2, device="cuda", dtype=torch.float32) / D))).contiguous()
+    cos, sin = rotary_tables(inv, q_pos[:, None])
+    q_out = torch.empty((B, 1, H, R, D), dtype=torch.bfloat16, device=device)
+    window = cap if ring else 0
+    kernels.kv_append(layers[1], k, v, write_pos=q_pos, flags=APPEND_FLAGS, q=q, q_out=q_out, q_norm_weight=w[0],
+                      k_norm_weight=w[1], rope_cos=cos, rope_sin=sin)
+    want = kernels.decode_attention(layers[1], q_out.view(B, H, R, D), km, q_pos=q_pos, window=window,
+                                    num_splits=_lib.G4_DECODE_TWO_PASS)
+    got = kernels.decode_attention_fused(layers[0], q[:, 0], km, q_pos=q_pos, window=window, k_raw=k[:, 0],
+                                         v_raw=v[:, 0], q_norm_weight=w[0], k_norm_weight=w[1], rope_cos=cos[:, 0],
+                                         rope_sin=sin[:, 0], eps=1e-6, flags=APPEND_FLAGS)
+    for a, b in ((got, want), (layers[0].key, layers[1].key), (layers[0].value_t, layers[1].value_t)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
