@@ -154,6 +154,14 @@ __device__ __forceinline__ u32x4 lds_read16(uint32_t addr) {
   return v;
 }
 
+// The same at addr + ofs, ofs in the instruction (a constant below 64 KiB once the caller's loop is
+// unrolled): one address register serves a whole run of tiles, with no add per read.
+__device__ __forceinline__ u32x4 lds_read16_at(uint32_t addr, int ofs) {
+  u32x4 v;
+  __asm__ volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "i"(ofs));
+  return v;
+}
+
 // s_waitcnt lgkmcnt(n), tied to `v` so that no use of v is scheduled before it (n a constant once
 // the caller's loop is unrolled; LDS reads complete in issue order).
 __device__ __forceinline__ void lgkm_wait(int n, u32x4& v) {

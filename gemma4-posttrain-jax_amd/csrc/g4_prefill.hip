@@ -205,47 +205,82 @@ __global__ __launch_bounds__(256) void prefill_f32_kernel(G4PrefillArgs a, int t
 
 constexpr int kLdsBytes = 160 * 1024;  // gfx950 LDS per workgroup
 
-// Two waves per SIMD, two 16-row column blocks each (measured per 32-key chunk against one wave per
-// SIMD with three or four blocks, which reuse each LDS tile more but leave a lone wave to overlap
-// its own MFMA, LDS and vector work: 1.85 ms vs 2.04 / 2.66 ms for the config-4 global layer).
-constexpr int kPfBlocks = 2;  // 16-row column blocks per wave
-constexpr int kPfWaves = 8;   // waves per workgroup
+// Two waves per SIMD, two 16-row column blocks each (measured per 32-key chunk at head dim 256 against
+// one wave per SIMD with three or four blocks, which reuse each LDS tile more but leave a lone wave to
+// overlap its own MFMA, LDS and vector work: 1.85 ms vs 2.04 / 2.66 ms for 8 x 4096 tokens). Head dim
+// 512 holds twice the q and output registers per column block: four waves of two blocks, one wave per
+// SIMD. At head dim 128 one block per wave takes 94 registers and 66 KiB of LDS, so two workgroups share
+// a CU and each fills the other's barriers (8 x 4096 tokens, causal 507 -> 479 us, window 512 178 ->
+// 148; 8 x 2000 192 -> 137).
+template <int D>
+constexpr int pf_blocks() { return D == 128 ? 1 : 2; }  // 16-row column blocks per wave
+template <int D>
+constexpr int pf_waves() { return D == 512 ? 4 : 8; }  // waves per workgroup
 
-// Largest key-mask row (bytes) the LDS-staged kernel of head dim 128 / 256 can hold next to its
+// Where two-block workgroups would leave CUs idle, one-block ones run instead, twice as many with
+// half the positions each and a shorter chunk step (2.55 -> 1.77 us per chunk at head dim 256, 3.6 ->
+// 2.4 at 512). Windowed rows: up to half the 256 CUs' count (1 x 4096 tokens, 2 kv heads, window 512:
+// 62.9 -> 45.5 us). Causal rows: up to the CU count, since the cost of a block grows with its position
+// and one round lasts as long as its last block, while two rounds pair long blocks with short ones
+// (1 x 1024: 88.9 -> 61.3 us; 4 x 1024 at head dim 512: 117.5 -> 84.9).
+constexpr int kPfFewGroups = 256;
+
+// Largest key-mask row (bytes) the LDS-staged kernel of head dim 128 / 256 / 512 can hold next to its
 // static tile buffers on each device; 0 when the limit could not be raised. Written once per device
 // by setup_prefill_kernels (under device_setup's std::call_once), read after it.
-int g_lds_max_seq[kMaxDevices][2];
+int g_lds_max_seq[kMaxDevices][3];
+
+template <int D>
+constexpr int pf_index() { return D == 512 ? 2 : D == 256; }
 
 template <int D>
 int raise_prefill_lds_limit(int device) {
-  int& max_seq = g_lds_max_seq[device][D == 256];
-  max_seq = 0;
-  hipFuncAttributes attr;
-  // a failed query or limit leaves max_seq at 0: every row then takes the register kernel
-  if (hipFuncGetAttributes(&attr, (const void*)prefill_bf16_lds_kernel<D, kPfBlocks, kPfWaves>) != hipSuccess) {
-    (void)hipGetLastError();
-    return G4_OK;
+  int& max_seq = g_lds_max_seq[device][pf_index<D>()];
+  max_seq = kPfMaxSeq;
+  const void* kernels[] = {(const void*)prefill_bf16_lds_kernel<D, 1, pf_waves<D>()>,
+                           (const void*)prefill_bf16_lds_kernel<D, pf_blocks<D>(), pf_waves<D>()>};
+  for (const void* fn : kernels) {
+    hipFuncAttributes attr;
+    int cap = 0;
+    // a failed query or limit leaves max_seq at 0: every row then takes the register kernel
+    if (hipFuncGetAttributes(&attr, fn) == hipSuccess)
+      cap = (kLdsBytes - (int)attr.sharedSizeBytes) / 16 * 16;
+    else
+      (void)hipGetLastError();
+    if (cap > kPfMaxSeq) cap = kPfMaxSeq;
+    if (cap <= 0 || !raise_lds_limit(device, fn, cap)) cap = 0;
+    if (cap < max_seq) max_seq = cap;
   }
-  const int room = (kLdsBytes - (int)attr.sharedSizeBytes) / 16 * 16;
-  const int cap = room < kPfMaxSeq ? room : kPfMaxSeq;
-  if (cap > 0 && raise_lds_limit(device, (const void*)prefill_bf16_lds_kernel<D, kPfBlocks, kPfWaves>, cap))
-    max_seq = cap;
   return G4_OK;
+}
+
+template <int D, int NB>
+void launch_prefill_blocks(const G4PrefillArgs& a, int64_t groups, hipStream_t st) {
+  const size_t lds = ((size_t)a.seq + 15) / 16 * 16;
+  hipLaunchKernelGGL((prefill_bf16_lds_kernel<D, NB, pf_waves<D>()>), dim3((unsigned)groups), dim3(pf_waves<D>() * 64),
+                     lds, st, a);
 }
 
 template <int D>
 void launch_prefill_lds(const G4PrefillArgs& a, hipStream_t st) {
-  const int ppb = kPfWaves * kPfBlocks * (16 / a.group);
-  const dim3 grid((unsigned)((a.seq + ppb - 1) / ppb) * (unsigned)a.kv_heads * (unsigned)a.batch);
-  const size_t lds = ((size_t)a.seq + 15) / 16 * 16;
-  hipLaunchKernelGGL((prefill_bf16_lds_kernel<D, kPfBlocks, kPfWaves>), grid, dim3(kPfWaves * 64), lds, st, a);
+  constexpr int NB = pf_blocks<D>();
+  const auto groups = [&](int nb) -> int64_t {  // workgroups of nb column blocks per wave
+    const int ppb = pf_waves<D>() * nb * (16 / a.group);
+    return (int64_t)((a.seq + ppb - 1) / ppb) * a.kv_heads * a.batch;
+  };
+  const bool causal = a.window <= 0 || a.window >= a.seq;
+  if (NB == 1 || groups(NB) <= (causal ? kPfFewGroups : kPfFewGroups / 2))
+    launch_prefill_blocks<D, 1>(a, groups(1), st);
+  else
+    launch_prefill_blocks<D, NB>(a, groups(NB), st);
 }
 
 }  // namespace
 
 int setup_prefill_kernels(int device) {
-  const int rc = raise_prefill_lds_limit<128>(device);
-  return rc != G4_OK ? rc : raise_prefill_lds_limit<256>(device);
+  int rc = raise_prefill_lds_limit<128>(device);
+  if (rc == G4_OK) rc = raise_prefill_lds_limit<256>(device);
+  return rc != G4_OK ? rc : raise_prefill_lds_limit<512>(device);
 }
 
 }  // namespace g4
@@ -273,7 +308,11 @@ extern "C" int g4_prefill_attention(const G4PrefillArgs* args, void* stream) {
     int dev = 0;
     const int rc = device_setup(&dev);
     if (rc != G4_OK) return rc;
-    // head dims 128/256: K/V chunks staged through LDS, when the row's key mask fits next to them
+    // head dims 128/256/512: K/V chunks staged through LDS, when the row's key mask fits next to them
+    if (a.head_dim == 512 && a.seq <= g_lds_max_seq[dev][2]) {
+      launch_prefill_lds<512>(a, st);
+      return check_launch("g4_prefill_attention");
+    }
     if (a.head_dim == 256 && a.seq <= g_lds_max_seq[dev][1]) {
       launch_prefill_lds<256>(a, st);
       return check_launch("g4_prefill_attention");

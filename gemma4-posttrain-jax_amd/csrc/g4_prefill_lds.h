@@ -1,12 +1,13 @@
-// bf16 prefill attention with the key / value chunks staged through LDS (head dims 128, 256);
+// bf16 prefill attention with the key / value chunks staged through LDS (head dims 128, 256, 512);
 // included by g4_prefill.hip after prefill_bf16_kernel.
 //
 // A workgroup of NW waves owns NW * NB * 16/R consecutive query positions of one (b, kv head);
 // each wave owns NB column blocks of 16 query rows (16/R positions x R heads each), so every K and
 // V^T operand tile it reads from LDS feeds NB MFMAs. The key range is walked in 32-key chunks:
 // every chunk's K and V^T are DMA'd into LDS once per workgroup (buffer_load ... lds, each wave
-// issuing an equal share, into rings of 4 slots) as lane-ordered MFMA operand tiles, and all waves
-// read them from there. The key-mask bytes of the row are staged in LDS once, so a chunk's validity
+// issuing an equal share, into rings of 4 slots, 2 at head dim 512, where a chunk's operand is 32 KiB)
+// as lane-ordered MFMA operand tiles, and all waves read them from there (head dim 512, 4 x 1024 tokens:
+// 600 us with one wave per SIMD loading its own operands, 97 us here). The key-mask bytes of the row are staged in LDS once, so a chunk's validity
 // is one LDS byte per lane and a ballot.
 //
 // Same two passes as prefill_bf16_kernel (the reference rounds probabilities after the full-row
@@ -34,6 +35,9 @@ template <int D, int NW>
 struct PfShape {
   static constexpr int KT = 2 * (D / 32);  // K operand tiles per chunk: (bb, s)
   static constexpr int VT = D / 16;        // V^T operand tiles per chunk: d-blocks
+  static constexpr int SLOTS = D >= 512 ? 2 : 4;  // ring slots of each operand in pass 2
+  static constexpr int CHUNK = KT * 1024;         // LDS bytes of a chunk's K (and V^T) tiles
+  static_assert(KT == VT, "K and V^T chunks share the ring");
   static constexpr int KT_W = KT / NW;     // DMA'd by each wave
   static constexpr int VT_W = VT / NW;
   static_assert(KT % NW == 0 && VT % NW == 0, "tiles split evenly over the waves");
@@ -56,18 +60,18 @@ __device__ __forceinline__ void pf_round8(const floatx4 (&acc)[2], float (&sc)[8
 }
 
 // S^T of one chunk for the wave's NB column blocks: K operand tiles (KT = 2 halves x KS d-slices,
-// 1 KiB each from LDS address kbase) against the q operands in registers, a rolling window of WIN
+// 1 KiB each, this lane's pieces from LDS address kbase) against the q operands in registers, a rolling window of WIN
 // tiles in flight (each read waited for right before its MFMAs; the chunk's DMA is covered by the
 // caller's vmcnt wait + barrier).
 template <int KT, int KS, int NB, int WIN>
-__device__ __forceinline__ void pf_qk(uint32_t kbase, const bf16x8 (&qop)[NB][KS], floatx4 (&acc)[NB][2], int lane) {
+__device__ __forceinline__ void pf_qk(uint32_t kbase, const bf16x8 (&qop)[NB][KS], floatx4 (&acc)[NB][2]) {
   static_assert(WIN >= 1 && WIN <= 8 && WIN <= KT, "window of LDS reads (lgkm_wait counts up to 7)");
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int cb = 0; cb < NB; ++cb) acc[cb][0] = acc[cb][1] = floatx4{0.f, 0.f, 0.f, 0.f};
   u32x4 kv[WIN];
 #pragma unroll
-  for (int j = 0; j < WIN; ++j) kv[j] = lds_read16(kbase + 1024u * j + 16u * lane);
+  for (int j = 0; j < WIN; ++j) kv[j] = lds_read16_at(kbase, 1024 * j);
 #pragma unroll
   for (int t = 0; t < KT; ++t) {
     const int bb = t / KS, s = t - bb * KS;
@@ -75,27 +79,27 @@ __device__ __forceinline__ void pf_qk(uint32_t kbase, const bf16x8 (&qop)[NB][KS
     lgkm_wait(later, kv[t % WIN]);
 #pragma unroll
     for (int cb = 0; cb < NB; ++cb) acc[cb][bb] = mfma16x16x32(as_bf16x8(kv[t % WIN]), qop[cb][s], acc[cb][bb]);
-    if (t + WIN < KT) kv[t % WIN] = lds_read16(kbase + 1024u * (t + WIN) + 16u * lane);
+    if (t + WIN < KT) kv[t % WIN] = lds_read16_at(kbase, 1024 * (t + WIN));
   }
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// O^T += V^T P^T over one chunk: VT value operand tiles (one per 16-dim block, 1 KiB each from LDS
-// address vbase) against the wave's probabilities, a rolling window of WIN tiles in flight.
+// O^T += V^T P^T over one chunk: VT value operand tiles (one per 16-dim block, 1 KiB each, this
+// lane's pieces from LDS address vbase) against the wave's probabilities, a rolling window of WIN tiles in flight.
 template <int VT, int NB, int WIN>
-__device__ __forceinline__ void pf_pv(uint32_t vbase, const bf16x8 (&pop)[NB], floatx4 (&oacc)[NB][VT], int lane) {
+__device__ __forceinline__ void pf_pv(uint32_t vbase, const bf16x8 (&pop)[NB], floatx4 (&oacc)[NB][VT]) {
   static_assert(WIN >= 1 && WIN <= 8 && WIN <= VT, "window of LDS reads (lgkm_wait counts up to 7)");
   __builtin_amdgcn_sched_barrier(0);
   u32x4 vv[WIN];
 #pragma unroll
-  for (int i = 0; i < WIN; ++i) vv[i] = lds_read16(vbase + 1024u * i + 16u * lane);
+  for (int i = 0; i < WIN; ++i) vv[i] = lds_read16_at(vbase, 1024 * i);
 #pragma unroll
   for (int i = 0; i < VT; ++i) {
     const int later = VT - 1 - i < WIN - 1 ? VT - 1 - i : WIN - 1;
     lgkm_wait(later, vv[i % WIN]);
 #pragma unroll
     for (int cb = 0; cb < NB; ++cb) oacc[cb][i] = mfma16x16x32(as_bf16x8(vv[i % WIN]), pop[cb], oacc[cb][i]);
-    if (i + WIN < VT) vv[i % WIN] = lds_read16(vbase + 1024u * (i + WIN) + 16u * lane);
+    if (i + WIN < VT) vv[i % WIN] = lds_read16_at(vbase, 1024 * (i + WIN));
   }
   __builtin_amdgcn_sched_barrier(0);
 }
@@ -104,16 +108,11 @@ template <int D, int NB, int NW>
 __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs a) {
   using S_ = PfShape<D, NW>;
   constexpr int KS = D / 32;
-  // the ring slots as separate arrays, so the compiler's wait before reading one does not include
-  // the DMA still in flight into the others
-  __shared__ __attribute__((aligned(1024))) unsigned char kb0[S_::KT][1024];
-  __shared__ __attribute__((aligned(1024))) unsigned char vb0[S_::VT][1024];
-  __shared__ __attribute__((aligned(1024))) unsigned char kb1[S_::KT][1024];
-  __shared__ __attribute__((aligned(1024))) unsigned char vb1[S_::VT][1024];
-  __shared__ __attribute__((aligned(1024))) unsigned char kb2[S_::KT][1024];
-  __shared__ __attribute__((aligned(1024))) unsigned char vb2[S_::VT][1024];
-  __shared__ __attribute__((aligned(1024))) unsigned char kb3[S_::KT][1024];
-  __shared__ __attribute__((aligned(1024))) unsigned char vb3[S_::VT][1024];
+  constexpr int SLOTS = S_::SLOTS;
+  // one array for the DMA's slots, read with inline-assembly LDS reads only: the compiler adds no
+  // waits of its own for the DMAs in flight (the key-mask bytes and the statistics are other arrays)
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[2 * SLOTS][S_::CHUNK];
+  __shared__ int first_valid[NW];
   extern __shared__ float smem[];
   uint8_t* km_lds = reinterpret_cast<uint8_t*>(smem);  // key_mask[b, 0:S]
 
@@ -179,34 +178,64 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
       qop[cb][s] = as_bf16x8(v);
     }
   }
+  // ... and the row's first valid key: the keys before it (a left-padded prompt's pads) score
+  // nothing, so the passes start at its chunk
   const uint8_t* km = a.key_mask + (int64_t)b * a.key_mask_stride;
-  for (int i = tid; i < S; i += blockDim.x) km_lds[i] = km[i];
+  int first = S;
+  for (int i = tid; i < S; i += blockDim.x) {
+    const uint8_t v = km[i];
+    km_lds[i] = v;
+    if (v && i < first) first = i;
+  }
+  // the q operands have landed here: waited for inside the loops, the compiler's count (it does not see
+  // the loops' own waits) would drain the DMAs in flight at every chunk
+#pragma unroll
+  for (int cb = 0; cb < NB; ++cb)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      u32x4 v = __builtin_bit_cast(u32x4, qop[cb][s]);
+      __asm__ volatile("" : "+v"(v));
+      qop[cb][s] = as_bf16x8(v);
+    }
+#pragma unroll
+  for (int msk = 32; msk >= 1; msk >>= 1) first = min(first, __shfl_xor(first, msk, 64));
+  if (lane == 0) first_valid[w] = first;
+  __syncthreads();  // key-mask bytes and first valid keys in LDS (no DMA in flight yet)
+#pragma unroll
+  for (int i = 0; i < NW; ++i) first = min(first, first_valid[i]);
+  first = __builtin_amdgcn_readfirstlane(first);
 
   const int pos_last = min(p0 + ppb - 1, S - 1);
-  const int kmin = a.window > 0 ? max(0, p0 - a.window + 1) : 0;
-  const int c_begin = kmin >> 5, c_end = pos_last >> 5;
+  const int kmin = max(first, a.window > 0 ? p0 - a.window + 1 : 0);
+  // chunks c_begin .. c_end hold every key a row of this workgroup may see (none: c_begin > c_end)
+  const int c_begin = kmin >> 5, c_end = kmin <= pos_last ? pos_last >> 5 : c_begin - 1;
 
   // This wave's share of a chunk's K / V^T operand tiles into LDS. Both layouts put chunk c at byte
-  // 64 * D * c, so a tile's lane offset does not depend on the chunk, which rides in soffset (every
-  // chunk issued lies inside the cache rows: c <= (S - 1) / 32 and S <= k_stride).
-  auto issue_k = [&](int c, unsigned char (&kt)[S_::KT][1024]) {
-    const uint32_t cofs = (uint32_t)c * (uint32_t)(64 * D);
+  // 64 * D * c; a tile's place in it is uniform too and rides in soffset with it, so each operand
+  // takes one lane offset (every chunk issued lies inside the cache rows: c <= (S - 1) / 32 and
+  // S <= k_stride).
+  const uint32_t k_lane = (uint32_t)(col * 64 + grp * 16);    // kt_index: lane col's 64-byte run, dims 8 grp ..
+  const uint32_t v_lane = vt_operand_bytes(grp, col, D);
+  auto issue_k = [&](int c, int slot) {
 #pragma unroll
     for (int i = 0; i < S_::KT_W; ++i) {
       const int t = w * S_::KT_W + i, bb = t / KS, s = t - bb * KS;
-      const uint32_t ko = (uint32_t)kt_index(8 * (col >> 2) + 4 * bb + (col & 3), 32 * s + 8 * grp, D) * 2u;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)&kt[t][0], 16, ko, cofs, 0, 0);
+      const uint32_t ofs = (uint32_t)c * (uint32_t)(64 * D) + (uint32_t)(2 * s + bb) * 1024u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (__attribute__((address_space(3))) void*)&ring[slot][1024 * t], 16,
+                                               k_lane, ofs, 0, 0);
     }
   };
-  auto issue_v = [&](int c, unsigned char (&vt)[S_::VT][1024]) {
-    const uint32_t cofs = (uint32_t)c * (uint32_t)(64 * D);
+  auto issue_v = [&](int c, int slot) {
 #pragma unroll
     for (int i = 0; i < S_::VT_W; ++i) {
       const int t = w * S_::VT_W + i;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (__attribute__((address_space(3))) void*)&vt[t][0], 16,
-                                               vt_operand_bytes(grp, 16 * t + col, D), cofs, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (__attribute__((address_space(3))) void*)&ring[slot][1024 * t], 16,
+                                               v_lane, (uint32_t)c * (uint32_t)(64 * D) + 256u * t, 0, 0);
     }
   };
+  // Hides the chunk index from the compiler, which would otherwise keep one register per lane for every
+  // bound of valid_bits and advance them from chunk to chunk (9 registers in pass 2: spills).
+  auto hide_chunk = [](int& c) { __asm__ volatile("" : "+s"(c)); };
   // key-mask ballot of the chunk's 32 keys (lanes l and l + 32 both hold key 32 c + l % 32)
   auto chunk_ballot = [&](int c) -> uint64_t {
     const int key = (c << 5) + (lane & 31);
@@ -244,9 +273,11 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
   }
   // one rescale per chunk: l <- l * exp(m - m') + sum exp(s - m') with m' = max(m, chunk max)
   // (masked keys score the fill value, whose exp vanishes against any real maximum)
-  auto stats = [&](int c, unsigned char (&kt)[S_::KT][1024]) {
+  const uint32_t ring0 = lds_addr(&ring[0][0]) + 16u * (uint32_t)lane;  // this lane's piece of a tile
+  auto stats = [&](int c, int slot) {
     floatx4 acc[NB][2];
-    pf_qk<S_::KT, KS, NB, 8>(lds_addr(&kt[0][0]), qop, acc, lane);  // pass 1 holds no value accumulators
+    pf_qk<S_::KT, KS, NB, 8>(ring0 + (uint32_t)(slot * S_::CHUNK), qop, acc);  // pass 1 holds no value accumulators
+    hide_chunk(c);
     const uint64_t mb = chunk_ballot(c);
     if (chunk_full(c, mb)) {
 #pragma unroll
@@ -292,30 +323,15 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
     else wait_vmcnt<0>();
     wg_barrier();
   };
-  __syncthreads();  // key-mask bytes in LDS (no DMA in flight yet)
-  issue_k(c_begin, kb0);
-  if (c_begin + 1 <= c_end) issue_k(c_begin + 1, kb1);
-  if (c_begin + 2 <= c_end) issue_k(c_begin + 2, kb2);
-  // (guarded steps rather than early exits: the accumulators then merge at one point per step)
-  for (int c = c_begin; c <= c_end; c += 4) {
+  // pass 1 rings through four slots whatever SLOTS is (the V^T slots are idle)
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    if (c_begin + j <= c_end) issue_k(c_begin + j, j);
+#pragma unroll 1
+  for (int c = c_begin, i = 0; c <= c_end; ++c, ++i) {
     wait_chunk(c, c_end);
-    if (c + 3 <= c_end) issue_k(c + 3, kb3);
-    stats(c, kb0);
-    if (c + 1 <= c_end) {
-      wait_chunk(c + 1, c_end);
-      if (c + 4 <= c_end) issue_k(c + 4, kb0);
-      stats(c + 1, kb1);
-    }
-    if (c + 2 <= c_end) {
-      wait_chunk(c + 2, c_end);
-      if (c + 5 <= c_end) issue_k(c + 5, kb1);
-      stats(c + 2, kb2);
-    }
-    if (c + 3 <= c_end) {
-      wait_chunk(c + 3, c_end);
-      if (c + 6 <= c_end) issue_k(c + 6, kb2);
-      stats(c + 3, kb3);
-    }
+    if (c + 3 <= c_end) issue_k(c + 3, (i + 3) & 3);
+    stats(c, i & 3);
   }
   bool row_masked[NB], mine_masked = false;
   float rl[NB];
@@ -335,9 +351,6 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
     rl[cb] = 1.0f / l[cb];
   }
   const bool any_masked = __syncthreads_or(mine_masked);  // (also: every wave is done with pass 1's LDS)
-  const float p_uniform = round_bf16(1.0f / (float)S);
-  const int c2_begin = any_masked ? 0 : c_begin;
-  const int c2_end = any_masked ? (S - 1) >> 5 : c_end;
 
   // ---- pass 2: exact probabilities and O^T = V^T P^T -------------------------------------------------
   floatx4 oacc[NB][S_::VT];
@@ -347,98 +360,152 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
     for (int i = 0; i < S_::VT; ++i) oacc[cb][i] = floatx4{0.f, 0.f, 0.f, 0.f};
   // exact bf16 probabilities of chunk c from its score accumulators (the B operand of O^T += V^T P^T)
   auto probs = [&](int c, const floatx4 (&acc)[NB][2], bf16x8 (&pop)[NB]) {
+    hide_chunk(c);
     const uint64_t mb = chunk_ballot(c);
-    if (!any_masked && chunk_full(c, mb)) {
-#pragma unroll
-      for (int cb = 0; cb < NB; ++cb) {
-        float sc[8], p[8];
-        pf_round8(acc[cb], sc);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) p[e] = __expf(sc[e] - m[cb]) * rl[cb];
-        pop[cb] = as_bf16x8(u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
-                                  pack_bf16x2(p[6], p[7])});
-      }
-      return;
-    }
-    const int kb = (c << 5) + 8 * grp;
+    const bool full = chunk_full(c, mb);
 #pragma unroll
     for (int cb = 0; cb < NB; ++cb) {
-      const uint32_t bits = valid_bits(c, mb, cb);
-      float p[8];
+      uint32_t pw[4];
+      if (full) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if (row_masked[cb]) p[e] = kb + e < S ? p_uniform : 0.f;
-        else p[e] = ((bits >> e) & 1u) ? __expf(round_bf16(acc[cb][e >> 2][e & 3]) - m[cb]) * rl[cb] : 0.f;
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t sw = pack_bf16x2(acc[cb][j >> 1][2 * (j & 1)], acc[cb][j >> 1][2 * (j & 1) + 1]);
+          pw[j] = pack_bf16x2(__expf(__uint_as_float(sw << 16) - m[cb]) * rl[cb],
+                              __expf(__uint_as_float(sw & 0xffff0000u) - m[cb]) * rl[cb]);
+        }
+        // (keeps the packing here: sunk below the branches, eight floats per block stay live over them)
+        __asm__ volatile("" : "+v"(pw[0]), "+v"(pw[1]), "+v"(pw[2]), "+v"(pw[3]));
+      } else {
+        const uint32_t bits = valid_bits(c, mb, cb);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t sw = pack_bf16x2(acc[cb][j >> 1][2 * (j & 1)], acc[cb][j >> 1][2 * (j & 1) + 1]);
+          const float p0 = __expf(__uint_as_float(sw << 16) - m[cb]) * rl[cb];
+          const float p1 = __expf(__uint_as_float(sw & 0xffff0000u) - m[cb]) * rl[cb];
+          pw[j] = pack_bf16x2((bits >> (2 * j)) & 1u ? p0 : 0.f, (bits >> (2 * j + 1)) & 1u ? p1 : 0.f);
+        }
       }
-      pop[cb] = as_bf16x8(u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
-                                pack_bf16x2(p[6], p[7])});
+      pop[cb] = as_bf16x8(u32x4{pw[0], pw[1], pw[2], pw[3]});
     }
   };
   // One barrier per chunk step. After the barrier of chunk c every wave runs two phases:
   // M(c) = the values of chunk c-1 (its V^T tiles x the probabilities formed earlier) and the QK of
   // chunk c (MFMA work), and P(c) = the probabilities of chunk c (VALU work). Waves 0..NW/2-1 run
-  // M(c) then P(c); waves NW/2.. run P(c-1) then M(c). Chunk j sits in slot (j - c2_begin) % 4 of
-  // both rings; K(c) and V(c-1) are read only in step c, and the barrier of chunk c queues K(c+3)
-  // and V(c+2) into the slots of K(c-1) and V(c-2), which step c-1 finished reading.
+  // M(c) then P(c); waves NW/2.. run P(c-1) then M(c). Chunk j sits in slot (j - c_begin) % SLOTS of
+  // both rings (K in slots 0 .. SLOTS-1, V^T behind them); K(c) and V(c-1) are read only in step c, and
+  // the barrier of chunk c queues K(c+SLOTS-1) and V(c+SLOTS-2) into the slots of K(c-1) and V(c-2),
+  // which step c-1 finished reading.
   const bool lead = w < NW / 2;
-  // this wave's DMAs of K(c) and V(c-1) have landed: queued after them are V(c) and, where they
-  // exist, K(c+1), K(c+2) and V(c+1)
+  // this wave's DMAs of K(c) and V(c-1) have landed: queued after them are, with four slots, V(c) and,
+  // where they exist, K(c+1), K(c+2) and V(c+1); with two slots nothing
   auto wait_step = [&](int c, int c_last) {
     constexpr int nk = S_::KT_W, nv = S_::VT_W;
-    if (c + 2 <= c_last) wait_vmcnt<2 * nk + 2 * nv>();
+    if (SLOTS == 2) wait_vmcnt<0>();
+    else if (c + 2 <= c_last) wait_vmcnt<2 * nk + 2 * nv>();
     else if (c + 1 <= c_last) wait_vmcnt<nk + 2 * nv>();
     else wait_vmcnt<nv>();
     wg_barrier();
   };
-  floatx4 acc[NB][2];
-  bf16x8 pop[NB];
-  auto p2_step = [&](int c, unsigned char (&kcur)[S_::KT][1024], unsigned char (&vprev)[S_::VT][1024],
-                     unsigned char (&knext)[S_::KT][1024], unsigned char (&vnext)[S_::VT][1024]) {
-    wait_step(c, c2_end);
-    if (c + 3 <= c2_end) issue_k(c + 3, knext);
-    if (c + 2 <= c2_end) issue_v(c + 2, vnext);
-    if (!lead && c > c2_begin) probs(c - 1, acc, pop);
-    __builtin_amdgcn_s_setprio(1);
-    if (c > c2_begin) pf_pv<S_::VT, NB, 4>(lds_addr(&vprev[0][0]), pop, oacc, lane);
-    pf_qk<S_::KT, KS, NB, 4>(lds_addr(&kcur[0][0]), qop, acc, lane);
-    __builtin_amdgcn_s_setprio(0);
-    if (lead) probs(c, acc, pop);
-  };
-  // prologue, in the steady state's order: K(b), K(b+1), V(b), K(b+2), V(b+1) (b = c2_begin <= c2_end:
-  // a row's own position is one of its keys)
-  issue_k(c2_begin, kb0);
-  if (c2_begin + 1 <= c2_end) issue_k(c2_begin + 1, kb1);
-  issue_v(c2_begin, vb0);
-  if (c2_begin + 2 <= c2_end) issue_k(c2_begin + 2, kb2);
-  if (c2_begin + 1 <= c2_end) issue_v(c2_begin + 1, vb1);
-  for (int c = c2_begin; c <= c2_end; c += 4) {  // guarded steps: the accumulators merge once per step
-    p2_step(c, kb0, vb3, kb3, vb2);
-    if (c + 1 <= c2_end) p2_step(c + 1, kb1, vb0, kb0, vb3);
-    if (c + 2 <= c2_end) p2_step(c + 2, kb2, vb1, kb1, vb0);
-    if (c + 3 <= c2_end) p2_step(c + 3, kb3, vb2, kb2, vb1);
-  }
-  // the last chunk's values: every wave's share of its V^T tiles has landed after this barrier
-  wait_vmcnt<0>();
-  wg_barrier();
-  if (!lead) probs(c2_end, acc, pop);
-  {
-    const int slot = (c2_end - c2_begin) & 3;
-    const uint32_t vlast = slot == 0   ? lds_addr(&vb0[0][0])
-                           : slot == 1 ? lds_addr(&vb1[0][0])
-                           : slot == 2 ? lds_addr(&vb2[0][0])
-                                       : lds_addr(&vb3[0][0]);
-    pf_pv<S_::VT, NB, 4>(vlast, pop, oacc, lane);
+  if (c_begin <= c_end) {  // (uniform over the workgroup)
+    floatx4 acc[NB][2];
+    bf16x8 pop[NB];
+    // prologue, in the steady state's order: K(b), then K(b+1), V(b), K(b+2), V(b+1) with four slots
+    issue_k(c_begin, 0);
+    if constexpr (SLOTS == 4) {
+      if (c_begin + 1 <= c_end) issue_k(c_begin + 1, 1);
+      issue_v(c_begin, SLOTS);
+      if (c_begin + 2 <= c_end) issue_k(c_begin + 2, 2);
+      if (c_begin + 1 <= c_end) issue_v(c_begin + 1, SLOTS + 1);
+    }
+#pragma unroll 1
+    for (int c = c_begin, i = 0; c <= c_end; ++c, ++i) {
+      wait_step(c, c_end);
+      if (c + SLOTS - 1 <= c_end) issue_k(c + SLOTS - 1, (i + SLOTS - 1) & (SLOTS - 1));
+      if (c + SLOTS - 2 <= c_end) issue_v(c + SLOTS - 2, SLOTS + ((i + SLOTS - 2) & (SLOTS - 1)));
+      if (!lead && c > c_begin) probs(c - 1, acc, pop);
+      __builtin_amdgcn_s_setprio(1);
+      if (c > c_begin)
+        pf_pv<S_::VT, NB, 4>(ring0 + (uint32_t)((SLOTS + ((i - 1) & (SLOTS - 1))) * S_::CHUNK), pop, oacc);
+      pf_qk<S_::KT, KS, NB, 4>(ring0 + (uint32_t)((i & (SLOTS - 1)) * S_::CHUNK), qop, acc);
+      __builtin_amdgcn_s_setprio(0);
+      if (lead) probs(c, acc, pop);
+    }
+    // the last chunk's values: every wave's share of its V^T tiles has landed after this barrier
+    wait_vmcnt<0>();
+    wg_barrier();
+    if (!lead) probs(c_end, acc, pop);
+    pf_pv<S_::VT, NB, 4>(ring0 + (uint32_t)((SLOTS + ((c_end - c_begin) & (SLOTS - 1))) * S_::CHUNK), pop, oacc);
   }
 
+  // the output row's address is computed here afresh (the lane is hidden from the compiler), not kept in
+  // registers over both passes since the q loads
+  int lane_o = lane;
+  __asm__ volatile("" : "+v"(lane_o));
+  auto out_row = [&](int cb) {
+    const int c = lane_o & 15, pos = p0 + w * ppw + cb * ppc + c / R;
+    return reinterpret_cast<uint16_t*>(a.out) + ((((int64_t)b * S + pos) * H + h) * R + c % R) * D;
+  };
 #pragma unroll
   for (int cb = 0; cb < NB; ++cb) {
-    if (row_ok[cb]) {
-      uint16_t* orow =
-          reinterpret_cast<uint16_t*>(a.out) + ((((int64_t)b * S + my_pos[cb]) * H + h) * R + r) * D;
+    if (row_ok[cb] && !row_masked[cb]) {
+      uint16_t* orow = out_row(cb);
 #pragma unroll
       for (int i = 0; i < S_::VT; ++i) {
         *reinterpret_cast<uint2*>(orow + 16 * i + 4 * grp) =
             make_uint2(pack_bf16x2(oacc[cb][i][0], oacc[cb][i][1]), pack_bf16x2(oacc[cb][i][2], oacc[cb][i][3]));
+      }
+    }
+  }
+
+  // ---- rows with no valid key: the average of all S values ------------------------------------------
+  // The reference's softmax over S equal fills is 1/S on every key, the same output for every such row
+  // of the pair. Wave w sums chunks w, w + NW, ... straight from memory (the same MFMA, the uniform
+  // probability in every column), the waves' sums meet in LDS, and each wave writes its masked rows:
+  // S D values read once per workgroup with a masked row, instead of both passes over all S keys (11
+  // prompts of 1999 left-padded tokens, window 512, with the pads' chunks skipped: 425 -> 177 us).
+  if (!any_masked) return;
+  float* usum = reinterpret_cast<float*>(&ring[0][0]);  // [NW][D], then the sum in row 0
+  const float p_uniform = round_bf16(1.0f / (float)S);
+  floatx4 uacc[S_::VT];
+#pragma unroll
+  for (int i = 0; i < S_::VT; ++i) uacc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int c = w; c <= (S - 1) >> 5; c += NW) {
+    float p[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) p[e] = (c << 5) + 8 * grp + e < S ? p_uniform : 0.f;
+    const bf16x8 pu = as_bf16x8(u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
+                                      pack_bf16x2(p[6], p[7])});
+    u32x4 v[S_::VT];
+#pragma unroll
+    for (int i = 0; i < S_::VT; ++i)
+      v[i] = buffer_load16(rv, v_lane, (uint32_t)c * (uint32_t)(64 * D) + 256u * i);
+    __builtin_amdgcn_sched_barrier(0);  // every load of the chunk requested before the first wait
+#pragma unroll
+    for (int i = 0; i < S_::VT; ++i) uacc[i] = mfma16x16x32(as_bf16x8(v[i]), pu, uacc[i]);
+  }
+  __syncthreads();  // every wave is done with the ring
+  if (col == 0) {
+#pragma unroll
+    for (int i = 0; i < S_::VT; ++i) *reinterpret_cast<floatx4*>(usum + w * D + 16 * i + 4 * grp) = uacc[i];
+  }
+  __syncthreads();
+  for (int d = tid; d < D; d += NW * 64) {
+    float t = usum[d];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) t += usum[i * D + d];
+    usum[d] = t;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int cb = 0; cb < NB; ++cb) {
+    if (row_masked[cb]) {
+      uint16_t* orow = out_row(cb);
+#pragma unroll
+      for (int i = 0; i < S_::VT; ++i) {
+        const floatx4 o = *reinterpret_cast<const floatx4*>(usum + 16 * i + 4 * grp);
+        *reinterpret_cast<uint2*>(orow + 16 * i + 4 * grp) =
+            make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
       }
     }
   }

@@ -1,0 +1,69 @@
+"""Prefill attention on the LDS-staged kernels where rows and grids can go wrong: rows without a valid key
+(pads, whole rows), key masks whose first valid key lies anywhere in a chunk, holes, and the grid sizes
+at which the number of column blocks per wave changes."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gemma4_posttrain_jax_amd import kernels
+from gemma4_posttrain_jax_amd.kvcache import group_keys, group_values
+from gpu_util import to_np
+from oracle import g4_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(device, B, S, H, R, D, window, key_mask, rows, seed):
+    """q and k scaled so that scores are of order 1: the outputs (|o| < 4) then differ from the oracle's
+    only by the rounding of probabilities and outputs, each at most half a bf16 ulp (2^-9 relative), plus
+    the f32 sums: below 2e-2."""
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g)  # noqa: E731
+    q = (rnd(B, S, H, R, D) * D ** -0.25).to(torch.bfloat16)
+    Sp = (S + 63) // 64 * 64
+    k = (rnd(B, H, Sp, D) * D ** -0.25).to(torch.bfloat16)
+    v = rnd(B, H, Sp, D).to(torch.bfloat16)
+    km = torch.from_numpy(key_mask).to(device)
+    out = to_np(kernels.prefill_attention(q, group_keys(k), group_values(v), km, window=window))
+    masks = O.make_qk_masks(key_mask, window if window else 1 << 30, 0, S)[O.SLIDING]
+    for b in rows:
+        want = O.attention_core(to_np(q[b:b + 1]).transpose(0, 1, 3, 2, 4), to_np(k[b:b + 1, :, :S]).transpose(0, 2, 1, 3),
+                                to_np(v[b:b + 1, :, :S]).transpose(0, 2, 1, 3), masks[b:b + 1], O.BF16)
+        err = np.abs(out[b] - want.transpose(0, 1, 3, 2, 4)[0]).max()
+        assert err <= 2e-2, f"row {b}: max |out - oracle| = {err}"
+
+
+@pytest.mark.parametrize("D", [128, 256, 512])
+@pytest.mark.parametrize("window", [0, 40])
+def test_prefill_masked_rows(device, D, window):
+    """Left pads that end on, before and after a chunk's and a workgroup's edge, every key masked, one
+    valid key, and holes, one wider than the window."""
+
+    S = 161
+    pads = [0, 1, 31, 32, 33, 64, 65, 128, 160, 161]
+    key_mask = np.arange(S)[None, :] >= np.array(pads + [0, 5])[:, None]
+    key_mask[-2, 40:100] = False
+    key_mask[-1, 6:160] = False
+    _check(device, len(key_mask), S, 1, 4, D, window, key_mask, range(len(key_mask)), D + window)
+
+
+# workgroups at two blocks per wave (64 positions at head dim 256, 32 at 512, R = 4): at and beyond 256
+# (causal) and 128 (windowed)
+@pytest.mark.parametrize("D,B,S,window", [(256, 32, 256, 0), (256, 32, 257, 0), (512, 32, 128, 0), (512, 32, 129, 0),
+                                          (256, 16, 256, 70), (256, 16, 257, 70), (512, 16, 128, 70),
+                                          (512, 16, 129, 70), (256, 8, 17, 0)])
+def test_prefill_block_count_lines(device, D, B, S, window):
+    key_mask = np.ones((B, S), bool)
+    key_mask[1, : S // 2] = False
+    _check(device, B, S, 2, 4, D, window, key_mask, (0, 1, B - 1), S + D)
+
+
+@pytest.mark.parametrize("D,R", [(512, 1), (512, 16), (256, 16), (256, 1)])
+def test_prefill_group_sizes_padded(device, D, R):
+    key_mask = np.ones((2, 100), bool)
+    key_mask[1, :37] = False
+    _check(device, 2, 100, 2, R, D, 0, key_mask, (0, 1), D + R)
