@@ -129,6 +129,19 @@ __device__ __forceinline__ void gemm_compute(const unsigned char* __restrict__ b
   }
 }
 
+// Waits until at most min(lines, MAX) lines' loads (G each) are outstanding.
+template <int G, int MAX>
+__device__ __forceinline__ void wait_lines(int lines) {
+  if constexpr (MAX > 0) {
+    if (lines >= MAX)
+      __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(MAX * G) : "memory");
+    else
+      wait_lines<G, MAX - 1>(lines);
+  } else {
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+}
+
 struct GemmLoop {
   __amdgpu_buffer_rsrc_t rx, rw;
   int K, kbeg, nst;
@@ -258,6 +271,241 @@ __global__ __launch_bounds__(GemmTile<TR>::THREADS) void linear_bf16_kernel(G4Li
   }
 }
 
+// --- few rows --------------------------------------------------------------------------------------
+//
+// A batch of a few rows only streams the weights: what counts is how many of their bytes are in flight
+// and how short the chain of one launch is, not the tile's reuse. A workgroup of NW waves owns 16 CB
+// columns x 8 XG rows of one K split; its waves divide the K range into 128-byte lines and each streams
+// its own lines of W and X into its own LDS slots (NBUF lines in flight), so there is no barrier until
+// the waves' partial sums meet in LDS at the end (added in wave order). The ring kernel above keeps one
+// stage sequence per workgroup, three stages ahead, and half its tile on padding rows here.
+// In HIP graphs over rotating weights (us; the ring kernel, for q/k/v and o hipBLASLt, before; now):
+//   rows   down, 8 K splits   q/k/v (N 3072)   o (N 2048)    K = 2048 (down 8192)
+//      1      12.0    7.3       11.3    4.2     11.0   4.0
+//     32      12.3    9.0       11.5    6.0     11.2   4.7
+//     64      12.8   11.0       11.9    7.1     11.7   5.7
+//    128      14.1 (ring)       14.4    9.1     11.1   6.7
+// (gate/up: launch_skinny_wide). Loaded straight into operand registers, the 16 rows of
+// an operand make every lane of an instruction a request of its own, 64 cycles per KiB instead of 16: q/k/v
+// at 32 rows 8.2 us. A load past a wave's last line costs the same time although it reads nothing, so
+// none is issued.
+constexpr int kSkinnyWaves = 4;
+// It takes every shape up to 64 rows, and beyond what one round of its largest tile covers (gate/up at
+// 128 rows takes two: 27.3 us against the ring kernel's 24.6).
+constexpr int kSkinnyRows = 64;
+constexpr int kSkinnyMaxCost = 16;
+constexpr int kSkinnyWideCols = 4096;  // columns from which one wave per column block fills the chip
+
+template <int NW, int CB, int XG, int NBUF, bool GELU>
+__global__ __launch_bounds__(NW * 64) void linear_skinny_kernel(G4LinearArgs a, float* partials) {
+  constexpr int MB = XG / 2, BLKS = CB * MB;
+  constexpr int GROUPS = 2 * CB + XG;  // DMA instructions (8 rows x 128 bytes) per line: W, then X
+  static_assert(!GELU || CB == 1 || CB % 2 == 0, "gate and up blocks in pairs, or halves of one block");
+  static_assert(BLKS <= NBUF * GROUPS, "the partial sums reuse the wave's slots");
+  static_assert((NBUF - 1) * GROUPS < 64, "vmcnt counts up to 63");
+  __shared__ __attribute__((aligned(1024))) unsigned char slots[NW][NBUF][GROUPS][kGroupBytes];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  // row groups of a (column tile, K split) unit go to one XCD, as in linear_bf16_kernel
+  const int n_rg = (a.m + 8 * XG - 1) / (8 * XG), n_units = a.n / (16 * CB) * a.ksplit;
+  const int j = (int)blockIdx.x >> 3;
+  const bool dealt = n_units % 8 == 0;
+  const int unit = dealt ? 8 * (j / n_rg) + ((int)blockIdx.x & 7) : (int)blockIdx.x / n_rg;
+  const int m0 = 8 * XG * (dealt ? j % n_rg : (int)blockIdx.x % n_rg);
+  const int tile = unit / a.ksplit, split = unit - tile * a.ksplit;
+  const int K = a.k, kper = K / a.ksplit;
+  const int lines = kper / 64;
+  const int s0 = lines * w / NW, cnt = lines * (w + 1) / NW - s0;  // this wave's lines
+  const int half = a.n / 2;
+  const uint32_t wbytes = (uint32_t)a.n * (uint32_t)K * 2u, xbytes = (uint32_t)a.m * (uint32_t)K * 2u;
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.w, wbytes), rx = make_rsrc(a.x, xbytes);
+  const uint32_t rl = (uint32_t)lane >> 3;
+  const uint32_t lane_ofs = rl * (uint32_t)K * 2u + (((uint32_t)lane & 7u) ^ rl) * 16u + (uint32_t)(split * kper) * 2u;
+
+  floatx4 acc[CB][MB];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[cb][mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  auto load = [&](int buf, int i) {
+    const uint32_t k2 = (uint32_t)(s0 + i) * 128u;
+#pragma unroll
+    for (int g = 0; g < 2 * CB; ++g) {
+      const int row = !GELU    ? tile * 16 * CB + 8 * g  // the first CB groups of a gated tile: gate rows
+                      : g < CB ? tile * 8 * CB + 8 * g
+                               : half + tile * 8 * CB + 8 * (g - CB);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void*)&slots[w][buf][g][0], 16,
+                                               lane_ofs + (uint32_t)row * (uint32_t)K * 2u + k2, 0, 0, kNonTemporal);
+    }
+#pragma unroll
+    for (int g = 0; g < XG; ++g)  // rows >= M: beyond the resource, zeros
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rx, (__attribute__((address_space(3))) void*)&slots[w][buf][2 * CB + g][0], 16,
+          lane_ofs + (uint32_t)(m0 + 8 * g) * (uint32_t)K * 2u + k2, 0, 0, 0);
+  };
+  const uint32_t slot0 = lds_addr(&slots[w][0][0][0]);
+  const int orow = col & 7;
+  const uint32_t opnd[2] = {slot0 + (uint32_t)((col >> 3) * kGroupBytes + (8 * orow + (grp ^ orow)) * 16),
+                            slot0 + (uint32_t)((col >> 3) * kGroupBytes + (8 * orow + ((4 + grp) ^ orow)) * 16)};
+  auto mac = [&](int buf) {
+    u32x4 wv[2][CB], xv[2][MB];
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+      const uint32_t at = opnd[kh] + (uint32_t)(buf * GROUPS * kGroupBytes);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) xv[kh][mb] = lds_read16_at(at, (2 * CB + 2 * mb) * kGroupBytes);
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) wv[kh][cb] = lds_read16_at(at, 2 * cb * kGroupBytes);
+    }
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) lgkm_wait(0, xv[kh][mb]);
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) lgkm_wait(0, wv[kh][cb]);
+    }
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          acc[cb][mb] = mfma16x16x32(as_bf16x8(wv[kh][cb]), as_bf16x8(xv[kh][mb]), acc[cb][mb]);
+  };
+  // line i sits in slot i % NBUF; while it is multiplied lines i + 1 .. i + NBUF - 1 are in flight. Its
+  // slot's operand reads have returned before the next line is requested into it.
+#pragma unroll
+  for (int i = 0; i < NBUF; ++i)
+    if (i < cnt) load(i, i);
+#pragma unroll 1
+  for (int i = 0; i < cnt; i += NBUF) {
+#pragma unroll
+    for (int u = 0; u < NBUF; ++u) {
+      if (i + u < cnt) {
+        // this line has landed; the lines requested after it, min(cnt - 1 - i - u, NBUF - 1), may not have
+        wait_lines<GROUPS, NBUF - 1>(cnt - 1 - (i + u));
+        mac(u);
+        if (i + u + NBUF < cnt) load(u, i + u + NBUF);
+      }
+    }
+  }
+  floatx4* red = reinterpret_cast<floatx4*>(&slots[w][0][0][0]);  // [BLKS][64] in this wave's own slots
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) red[(cb * MB + mb) * 64 + lane] = acc[cb][mb];
+  __syncthreads();
+
+  // quad q: block q / 64, lane q % 64 of the MFMA result: Y[m = m0 + 16 mb + col][4 consecutive columns]
+  auto sum = [&](int blk, int l) {
+    floatx4 t = reinterpret_cast<const floatx4*>(&slots[0][0][0][0])[blk * 64 + l];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) t += reinterpret_cast<const floatx4*>(&slots[i][0][0][0])[blk * 64 + l];
+    return t;
+  };
+  // (gated GELU: the up quad of a gate quad is CB / 2 column blocks on; with CB = 1, rows 0 .. 7 of the
+  // block are gate rows and 8 .. 15 their up rows, 32 lanes on)
+  constexpr int QL = GELU && CB == 1 ? 32 : 64;
+  constexpr int QUADS = GELU && CB > 1 ? BLKS / 2 * 64 : BLKS * QL;
+  for (int q = threadIdx.x; q < QUADS; q += NW * 64) {
+    const int blk = q / QL, l = q % QL, cb = blk / MB, mb = blk - cb * MB;
+    const int m = m0 + 16 * mb + (l & 15);
+    if (m >= a.m) continue;
+    const floatx4 t = sum(blk, l);
+    if (GELU) {
+      const floatx4 up = CB == 1 ? sum(blk, l + 32) : sum(blk + BLKS / 2, l);
+      float y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = gelu_tanh_mul(round_bf16(t[j]), round_bf16(up[j]));
+      uint16_t* dst = reinterpret_cast<uint16_t*>(a.y) + (int64_t)m * a.ldy + tile * 8 * CB + 16 * cb + 4 * (l >> 4);
+      *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+    } else {
+      const int n = tile * 16 * CB + 16 * cb + 4 * (l >> 4);
+      if (a.ksplit == 1) {
+        uint16_t* dst = reinterpret_cast<uint16_t*>(a.y) + (int64_t)m * a.ldy + n;
+        *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(t[0], t[1]), pack_bf16x2(t[2], t[3]));
+      } else {
+        *reinterpret_cast<floatx4*>(partials + ((int64_t)split * a.m + m) * a.n + n) = t;
+      }
+    }
+  }
+}
+
+// LDS slots per wave (lines in flight): what lets two workgroups share a CU where a line is small
+// (64 - 80 KiB; (CB 2, XG 4): 2 slots 14.5 us, 4 slots 16.2 for gate/up at 32 rows), else all of it. A
+// one-wave workgroup takes 40 KiB, four to a CU (80 KiB: 24576 columns at 16 rows 28.8 -> 36.5 us).
+template <int NW, int CB, int XG>
+constexpr int skinny_slots() {
+  if (NW == 1) return 40 / (2 * CB + XG);
+  return CB == 1 ? (XG == 2 ? 4 : XG == 4 ? 3 : 2) : CB == 2 ? (XG == 4 ? 2 : 3) : (XG == 8 ? 2 : 3);
+}
+
+template <int NW, int CB, int XG>
+void launch_skinny(const G4LinearArgs& a, float* partials, hipStream_t st) {
+  constexpr int NBUF = skinny_slots<NW, CB, XG>();
+  const int n_rg = (a.m + 8 * XG - 1) / (8 * XG);
+  const dim3 grid((unsigned)(a.n / (16 * CB) * a.ksplit * n_rg)), block(NW * 64);
+  if constexpr (CB % 2 == 0 || NW == 1)
+    if (a.epilogue == G4_LINEAR_GELU_MUL) {
+      hipLaunchKernelGGL((linear_skinny_kernel<NW, CB, XG, NBUF, true>), grid, block, 0, st, a, partials);
+      return;
+    }
+  hipLaunchKernelGGL((linear_skinny_kernel<NW, CB, XG, NBUF, false>), grid, block, 0, st, a, partials);
+}
+
+// Many columns, one K range (gate/up): one wave per workgroup walks all of K for its 16 CB columns, so the
+// sums keep the ring kernel's order (split over four waves the 16384 columns take 12.9 us instead of 15.9
+// at 16 rows, but the gated GELU's roundings then move 3e-4 of the MLP's output). One column block per
+// wave while that leaves at most two per CU, else two (gate/up + GELU, K = 2048, us at 1 / 16 / 64 rows,
+// ring kernel, now: 4096 columns 18.3 / 18.2 / 19.9, 7.5 / 7.7 / 11.1; 8192 19.0 / 19.0 / 20.8, 9.6 / 9.2 /
+// 13.0; 16384 21.8 / 21.7 / 23.5, 16.3 / 15.9 / 19.3; 24576 x 3072 54 / 52 / 56, 28 / 29 / 40).
+template <int CB>
+void launch_skinny_wide(const G4LinearArgs& a, float* partials, hipStream_t st) {
+  if (a.m <= 16)
+    launch_skinny<1, CB, 2>(a, partials, st);
+  else if (a.m <= 32)
+    launch_skinny<1, CB, 4>(a, partials, st);
+  else
+    launch_skinny<1, CB, 8>(a, partials, st);
+}
+
+// The tile (16 CB columns x 8 XG rows) whose workgroups bring the least through each of the 256 CUs:
+// cost = ceil(workgroups / 256) x (2 CB + XG) KiB per line.
+struct SkinnyTile {
+  int cb, xg;
+  int64_t cost;
+};
+
+SkinnyTile skinny_tile(const G4LinearArgs& a, bool gelu) {
+  SkinnyTile best = {0, 0, 0};
+  for (int cb = gelu ? 2 : 1; cb <= 4; cb *= 2)
+    for (int xg = 2; xg <= 8; xg *= 2) {
+      if (xg > 2 && 4 * xg >= a.m) break;  // half the rows would do
+      const int64_t groups = (int64_t)(a.n / (16 * cb)) * a.ksplit * ((a.m + 8 * xg - 1) / (8 * xg));
+      // (4, 2) leaves one workgroup per CU, whose last lines nothing overlaps: gate/up at 16 rows 13.4 us
+      // against 12.9 with two (2, 2) workgroups per CU
+      const int64_t cost = (groups + 255) / 256 * (2 * cb + xg) + (cb == 4 && xg == 2 ? 3 : 0);
+      if (!best.cb || cost < best.cost) best = {cb, xg, cost};
+    }
+  return best;
+}
+
+void launch_skinny_tile(const SkinnyTile& t, const G4LinearArgs& a, float* partials, hipStream_t st) {
+  switch (t.cb * 16 + t.xg) {
+    case 16 + 2: return launch_skinny<kSkinnyWaves, 1, 2>(a, partials, st);
+    case 16 + 4: return launch_skinny<kSkinnyWaves, 1, 4>(a, partials, st);
+    case 16 + 8: return launch_skinny<kSkinnyWaves, 1, 8>(a, partials, st);
+    case 32 + 2: return launch_skinny<kSkinnyWaves, 2, 2>(a, partials, st);
+    case 32 + 4: return launch_skinny<kSkinnyWaves, 2, 4>(a, partials, st);
+    case 32 + 8: return launch_skinny<kSkinnyWaves, 2, 8>(a, partials, st);
+    case 64 + 2: return launch_skinny<kSkinnyWaves, 4, 2>(a, partials, st);
+    case 64 + 4: return launch_skinny<kSkinnyWaves, 4, 4>(a, partials, st);
+    default: return launch_skinny<kSkinnyWaves, 4, 8>(a, partials, st);
+  }
+}
+
 // Y = sum of the split partials (split order), rounded to bf16; 4 outputs per thread.
 __global__ __launch_bounds__(256) void linear_reduce_kernel(G4LinearArgs a, const float* partials) {
   const int64_t i4 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
@@ -306,8 +554,18 @@ extern "C" int g4_linear_bf16(const G4LinearArgs* args, void* stream) {
                 a.workspace ? a.workspace_bytes : (size_t)0);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   float* partials = reinterpret_cast<float*>(a.workspace);
-  // 128 x 128 tiles when the rows fill two halves and the columns divide by 128; else 256 x 64
-  if (a.m > 128 && a.n % 128 == 0)
+  // few rows: the streaming kernel (neither the choice nor the order of the sums depends on the epilogue:
+  // the gated GELU's products are the plain call's bit for bit); else 128 x 128 tiles when the rows fill
+  // two halves and the columns divide by 128; else 256 x 64
+  const bool wide = a.n >= kSkinnyWideCols && a.ksplit == 1;
+  if (wide && a.m <= kSkinnyRows) {
+    if (a.n / 16 <= 512)
+      launch_skinny_wide<1>(a, partials, st);
+    else
+      launch_skinny_wide<2>(a, partials, st);
+  } else if (!wide && (a.m <= kSkinnyRows || skinny_tile(a, false).cost <= kSkinnyMaxCost))
+    launch_skinny_tile(skinny_tile(a, a.epilogue == G4_LINEAR_GELU_MUL), a, partials, st);
+  else if (a.m > 128 && a.n % 128 == 0)
     hipLaunchKernelGGL(linear_bf16_kernel<128>, dim3((unsigned)(a.n / 128 * a.ksplit * 2)), dim3(GemmTile<128>::THREADS), 0,
                        st, a, partials);
   else

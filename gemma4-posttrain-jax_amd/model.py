@@ -256,10 +256,26 @@ def _mm(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     return a @ b
 
 
-def _proj(x: torch.Tensor, w_t: torch.Tensor) -> torch.Tensor:
-    """``x [T, K] . w_t[N, K]^T`` in x's dtype (hipBLASLt; the [N, K] weight layout is its faster
-    one for the prefill shapes and equal at decode)."""
+def _native_proj(x: torch.Tensor, w_t: torch.Tensor) -> bool:
+    """Whether a projection runs as g4_linear_bf16: a bf16 decode batch of at most 192 rows, and shapes its
+    few-row kernel streams in one round (every shape up to 64 rows). At 256 rows the library's tiles fill
+    (q/k/v 13.0 / 12.0 us, o 11.6 / 8.8) and it stays: 1 % of that step, for outputs that round from
+    another f32 order."""
 
+    (rows, k), n = x.shape, w_t.shape[0]
+    return (x.is_cuda and x.dtype == torch.bfloat16 and w_t.dtype == torch.bfloat16 and 0 < rows <= 192
+            and (rows <= 64 or (k <= 4096 and n < 4096)) and n % 64 == 0 and k % 64 == 0
+            and n * k < 2 ** 30 and x.is_contiguous() and w_t.is_contiguous())
+
+
+def _proj(x: torch.Tensor, w_t: torch.Tensor) -> torch.Tensor:
+    """``x [T, K] . w_t[N, K]^T`` in x's dtype: the native few-row GEMM for a decode batch (at K = 2048,
+    N = 3072 / 2048: 11.3 / 11.0 us in hipBLASLt, 4.3 / 4.1 native at 1 row, 11.9 / 11.7 and 7.1 / 5.7 at
+    64, 14.4 / 11.1 and 9.0 / 6.7 at 128), hipBLASLt beyond (the [N, K] weight layout is its faster one
+    for the prefill shapes)."""
+
+    if _native_proj(x, w_t):
+        return kernels.linear(x, w_t)
     return _mm(x, w_t.t())
 
 

@@ -66,3 +66,30 @@ def test_fused_preparation_of_one_row(device, R, ring, cap):
                                          rope_sin=sin[:, 0], eps=1e-6, flags=APPEND_FLAGS)
     for a, b in ((got, want), (layers[0].key, layers[1].key), (layers[0].value_t, layers[1].value_t)):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+# rows at the edges of the row groups and of the tile choice, K ranges that leave waves without a line
+# (64, 192), that do not divide among the waves (576) and that fill every slot; the bars as in
+# test_gpu_linear: half a bf16 ulp of the f32-accumulated sum (the split sums are not rounded), and for the
+# gated GELU the roundings of g, u and the product
+@pytest.mark.parametrize("rows", [1, 16, 17, 33, 64, 65, 128, 192])
+@pytest.mark.parametrize("n,k", [(64, 64), (128, 192), (320, 576), (3072, 2048), (4096, 640), (8256, 192)])
+def test_few_row_linear(device, rows, n, k):
+    g = torch.Generator(device="cuda").manual_seed(rows + n + k)
+    x = torch.randn((rows, k), device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn((n, k), device="cuda", generator=g) * k ** -0.5).to(torch.bfloat16)
+    ref = x.double() @ w.double().T
+    slack = 2.0 ** -20 * (x.double().abs() @ w.double().abs().T)  # f32 sums of k products in any order
+    out = torch.full((rows, n + 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    y = kernels.linear(x, w, out=out[:, :n])
+    assert torch.all((y.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + slack)
+    assert torch.isnan(out[:, n:].float()).all()  # columns past n untouched
+    if k % 192 == 0:
+        parts = kernels.linear_partials(x, w, ksplit=3)
+        assert torch.all((parts.double().sum(0) - ref).abs() <= slack)
+    gate, up = (t.to(torch.bfloat16).double() for t in ref.chunk(2, -1))
+    want = torch.nn.functional.gelu(gate, approximate="tanh") * up
+    got = kernels.linear_gelu(x, w).double()
+    # g and u one rounding apart at most (2^-8 relative each, gelu'(g) <= 1.13 and gelu(g) ~ g / 2 below)
+    bar = 2.0 ** -7 * (want.abs() + 1.2 * gate.abs() * up.abs()) + 2.0 * slack.chunk(2, -1)[0] * up.abs() + 1e-6
+    assert torch.all((got - want).abs() <= bar)
