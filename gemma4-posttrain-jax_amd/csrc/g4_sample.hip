@@ -214,6 +214,7 @@ __global__ void advance_key_kernel(uint32_t* key) {
 // advance_key_kernel.
 constexpr int kTkMaxK = 256;
 constexpr int kTkCand = 2048;
+constexpr int kTkRedo = (int)0x80000000;  // token of a row left to the general kernel
 
 __device__ __forceinline__ uint32_t score_key(float s) {
   uint32_t u = __float_as_uint(s == 0.f ? 0.f : s);
@@ -261,7 +262,104 @@ __device__ __forceinline__ float pairwise_sum_f32(const float* a, int n) {
   return pairwise_block_f32(a, n2) + right;
 }
 
-template <bool BF16, bool VEC>
+// Candidates (n_cand of them, at least K) -> the drawn token and its log-probability: steps 2 (ranking)
+// and 3 above. m and sum: the row's log-softmax state. Arrays in LDS; `w` may alias the candidates.
+struct TkProposal {
+  float s[kTkMaxK];
+  int32_t id[kTkMaxK];
+  float x[kTkMaxK];
+  float best[kSampleThreads / 64];
+  int best_j[kSampleThreads / 64];
+};
+
+__device__ __forceinline__ void tk_draw(const G4SampleTopKArgs& a, int row, const uint32_t* cand_key,
+                                        const int32_t* cand_id, float* cand_x, uint32_t n_cand, float m, float sum,
+                                        TkProposal& prop) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int K = a.top_k;
+  float* prop_s = prop.s;
+  int32_t* prop_id = prop.id;
+  float* prop_x = prop.x;
+  float* s_best = prop.best;
+  int* s_best_j = prop.best_j;
+  // ---- the sorted proposal: rank of each candidate among them ------------------------------------
+  for (int e = tid; e < (int)n_cand; e += kSampleThreads) {
+    const uint32_t ke = cand_key[e];
+    const int ie = cand_id[e];
+    int r = 0;
+    for (int j = 0; j < (int)n_cand; ++j) {
+      const uint32_t kj = cand_key[j];
+      r += (kj > ke) || (kj == ke && cand_id[j] < ie);
+    }
+    if (r < K) {
+      prop_s[r] = key_score(ke);
+      prop_id[r] = ie;
+      prop_x[r] = cand_x[e];
+    }
+  }
+  __syncthreads();
+
+  // ---- top-p over the proposal --------------------------------------------------------------------
+  if (a.top_p < 1.f) {
+    float* w = reinterpret_cast<float*>(cand_x);  // reused: the candidates are in the proposal now
+    if (tid < K) w[tid] = expf(prop_s[tid] - prop_s[0]);
+    __syncthreads();
+    if (tid == 0) {
+      const float total = pairwise_sum_f32(w, K);
+      float cum = 0.f;
+      for (int j = 0; j < K; ++j) {
+        const float prob = w[j] / total;
+        if (j > 0 && !(cum < a.top_p)) prop_s[j] = -INFINITY;  // the mass before column j
+        cum += prob;
+      }
+    }
+    __syncthreads();
+  }
+
+  // ---- categorical over the K columns ------------------------------------------------------------
+  uint32_t k0 = a.key[0], k1 = a.key[1];
+  if (a.split_key) {  // sample_key = split(key)[1] = threefry2x32(key, (0, 1))
+    uint32_t x0 = 0u, x1 = 1u;
+    threefry2x32(k0, k1, x0, x1);
+    k0 = x0;
+    k1 = x1;
+  }
+  float best = -INFINITY;
+  int best_j = 0x7fffffff;
+  if (tid < K) {
+    best = prop_s[tid] + gumbel(k0, k1, (uint64_t)row * (uint64_t)K + (uint64_t)tid);
+    best_j = tid;
+  }
+#pragma unroll
+  for (int msk = 32; msk >= 1; msk >>= 1) {
+    const float ob = __shfl_xor(best, msk, 64);
+    const int oj = __shfl_xor(best_j, msk, 64);
+    if (beats(ob, oj, best, best_j)) {
+      best = ob;
+      best_j = oj;
+    }
+  }
+  if (lane == 0) {
+    s_best[wv] = best;
+    s_best_j[wv] = best_j;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    float b = s_best[0];
+    int j = s_best_j[0];
+    for (int i = 1; i < (K + 63) / 64; ++i)
+      if (beats(s_best[i], s_best_j[i], b, j)) {
+        b = s_best[i];
+        j = s_best_j[i];
+      }
+    j = j < 0 ? 0 : (j >= K ? K - 1 : j);
+    a.token_out[row] = prop_id[j];
+    a.logp_out[row] = (prop_x[j] - m) - logf(sum);
+  }
+}
+
+// REDO: only the rows that sample_top_k_hist_kernel marked.
+template <bool BF16, bool VEC, bool REDO = false>
 __global__ __launch_bounds__(kSampleThreads) void sample_top_k_kernel(G4SampleTopKArgs a) {
   using T = typename Elem<BF16>::T;
   __shared__ uint16_t cap_tab[BF16 ? kCapTableEntries : 1];
@@ -270,16 +368,13 @@ __global__ __launch_bounds__(kSampleThreads) void sample_top_k_kernel(G4SampleTo
   __shared__ uint32_t cand_key[kTkCand];
   __shared__ int32_t cand_id[kTkCand];
   __shared__ float cand_x[kTkCand];
-  __shared__ float prop_s[kTkMaxK];
-  __shared__ int32_t prop_id[kTkMaxK];
-  __shared__ float prop_x[kTkMaxK];
+  __shared__ TkProposal prop;
   __shared__ RowState red[kSampleThreads / 64];
   __shared__ uint32_t scan[kSampleThreads];
   __shared__ uint32_t s_count, s_bin, s_need;
-  __shared__ float s_best[kSampleThreads / 64];
-  __shared__ int s_best_j[kSampleThreads / 64];
 
   const int row = blockIdx.x;
+  if (REDO && a.token_out[row] != kTkRedo) return;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int V = a.vocab, K = a.top_k;
   const CapTable ct = cap_table(cap_tab, a.softcap);
@@ -517,80 +612,203 @@ __global__ __launch_bounds__(kSampleThreads) void sample_top_k_kernel(G4SampleTo
     n_cand = (uint32_t)K;
   }
 
-  // ---- the sorted proposal: rank of each candidate among them ------------------------------------
-  for (int e = tid; e < (int)n_cand; e += kSampleThreads) {
-    const uint32_t ke = cand_key[e];
-    const int ie = cand_id[e];
-    int r = 0;
-    for (int j = 0; j < (int)n_cand; ++j) {
-      const uint32_t kj = cand_key[j];
-      r += (kj > ke) || (kj == ke && cand_id[j] < ie);
-    }
-    if (r < K) {
-      prop_s[r] = key_score(ke);
-      prop_id[r] = ie;
-      prop_x[r] = cand_x[e];
-    }
-  }
-  __syncthreads();
+  tk_draw(a, row, cand_key, cand_id, cand_x, n_cand, full.m, full.s, prop);
+}
 
-  // ---- top-p over the proposal --------------------------------------------------------------------
-  if (a.top_p < 1.f) {
-    float* w = reinterpret_cast<float*>(cand_x);  // reused: the candidates are in the proposal now
-    if (tid < K) w[tid] = expf(prop_s[tid] - prop_s[0]);
-    __syncthreads();
-    if (tid == 0) {
-      const float total = pairwise_sum_f32(w, K);
-      float cum = 0.f;
-      for (int j = 0; j < K; ++j) {
-        const float prob = w[j] / total;
-        if (j > 0 && !(cum < a.top_p)) prop_s[j] = -INFINITY;  // the mass before column j
-        cum += prob;
+// The same draw for a bf16 row of a large vocabulary (VEC rows). A bf16 logit has 65536 values, so one
+// pass counts them in LDS (16-bit counters, order-preserving index, non-negative values in the high halves
+// and negative ones in the low halves of 32768 words): five VALU instructions and one LDS add per column
+// instead of the soft-cap, exp and insertion of the general kernel (about 85). From the counts come the
+// log-softmax sum (one exp per distinct value), the value that holds the k-th largest score and, since the
+// soft-cap and the division are monotone, the smallest logit whose score ties with it; a second pass over
+// the row (from the Infinity Cache) gathers every column at or above that logit. A row that does not fit
+// the scheme -- a value met more than 65535 times, NaNs, more than kTkCand candidates, over 1024 distinct
+// logits tied with the k-th score -- is marked kTkRedo and drawn by the general kernel, launched behind.
+// k = 50, general kernel, this one (us): V = 262144 164 / 54 at 64 rows, 181 / 67 at 256; V = 32768 73 / 31;
+// V = 4096 57 / 27.
+constexpr int kTkHistVocab = 4096;  // smallest vocabulary
+
+__device__ __forceinline__ uint32_t order2(uint32_t w) {  // both bf16 halves -> order-preserving 16-bit indexes
+  return w ^ ((((w >> 15) & 0x00010001u) * 0x7fffu) | 0x80008000u);
+}
+
+__device__ __forceinline__ uint32_t order_bits(uint32_t o) {  // index -> bf16 bits
+  return o & 0x8000u ? o ^ 0x8000u : o ^ 0xffffu;
+}
+
+__global__ __launch_bounds__(kSampleThreads) void sample_top_k_hist_kernel(G4SampleTopKArgs a) {
+  __shared__ __attribute__((aligned(16))) uint32_t hist[32768];
+  __shared__ uint32_t blk[64];  // elements per 1024 consecutive indexes
+  __shared__ uint32_t wmax[kSampleThreads / 64], wcnt[kSampleThreads / 64];
+  __shared__ double wsum[kSampleThreads / 64];
+  __shared__ uint32_t s_count, s_index, s_fail, s_block, s_above;
+  __shared__ TkProposal prop;
+  constexpr int NW = kSampleThreads / 64;
+  const int row = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int V = a.vocab, K = a.top_k;
+  const uint16_t* lrow = reinterpret_cast<const uint16_t*>(a.logits) + (int64_t)row * a.row_stride;
+  const int nchunks = V / 8;
+  const bool unit_t = a.temperature == 1.0f;
+  auto capped_x = [&](uint32_t o) {
+    const float x = bf16_bits_to_f32(order_bits(o));
+    return a.softcap > 0.f ? softcap_formula(x, a.softcap) : x;
+  };
+  auto key_of = [&](float x) { return score_key(unit_t ? x : x / a.temperature); };
+  // every 16-byte chunk of the row (8 columns), four requested at a time: f(chunk index, its words)
+  auto each_chunk = [&](auto&& f) {
+    for (int j0 = tid; j0 - lane < nchunks; j0 += 4 * kSampleThreads) {
+      u32x4 r[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int j = j0 + u * kSampleThreads;
+        r[u] = j < nchunks ? *reinterpret_cast<const u32x4*>(lrow + 8 * j) : u32x4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) f(j0 + u * kSampleThreads, r[u]);
+    }
+  };
+
+  // ---- counts ------------------------------------------------------------------------------------
+  for (int i = tid; i < 32768 / 4; i += kSampleThreads) reinterpret_cast<u32x4*>(hist)[i] = u32x4{0u, 0u, 0u, 0u};
+  if (tid < 64) blk[tid] = 0u;
+  if (tid == 0) s_count = s_fail = 0u;
+  __syncthreads();
+  each_chunk([&](int j, u32x4 r) {
+    if (j < nchunks) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t o = order2(r[q]);
+        atomicAdd(&hist[o & 0x7fffu], o & 0x8000u ? 0x10000u : 1u);
+        atomicAdd(&hist[(o >> 16) & 0x7fffu], o & 0x80000000u ? 0x10000u : 1u);
       }
     }
-    __syncthreads();
-  }
+  });
+  __syncthreads();
 
-  // ---- categorical over the K columns ------------------------------------------------------------
-  uint32_t k0 = a.key[0], k1 = a.key[1];
-  if (a.split_key) {  // sample_key = split(key)[1] = threefry2x32(key, (0, 1))
-    uint32_t x0 = 0u, x1 = 1u;
-    threefry2x32(k0, k1, x0, x1);
-    k0 = x0;
-    k1 = x1;
-  }
-  float best = -INFINITY;
-  int best_j = 0x7fffffff;
-  if (tid < K) {
-    best = prop_s[tid] + gumbel(k0, k1, (uint64_t)row * (uint64_t)K + (uint64_t)tid);
-    best_j = tid;
+  // ---- per thread: words tid + 1024 i. Block totals, the largest index, NaNs ----------------------
+  uint32_t top = 0u;
+  bool nan = false;
+  for (int i = 0; i < 32; ++i) {
+    const uint32_t c = hist[tid + kSampleThreads * i];
+    if (__ballot(c != 0u) == 0ull) continue;
+    const uint32_t o = (uint32_t)(tid + kSampleThreads * i);
+    const uint32_t lo = c & 0xffffu, hi = c >> 16;
+    if (hi) top = max(top, o + 0x8000u);
+    else if (lo) top = max(top, o);
+    nan = nan || (hi && o + 0x8000u > 0xff80u) || (lo && o < 0x007fu);
+    const uint32_t tl = (uint32_t)__reduce_add_sync(~0ull, lo), th = (uint32_t)__reduce_add_sync(~0ull, hi);
+    if (lane == 0) {
+      if (tl) atomicAdd(&blk[i], tl);
+      if (th) atomicAdd(&blk[32 + i], th);
+    }
   }
 #pragma unroll
-  for (int msk = 32; msk >= 1; msk >>= 1) {
-    const float ob = __shfl_xor(best, msk, 64);
-    const int oj = __shfl_xor(best_j, msk, 64);
-    if (beats(ob, oj, best, best_j)) {
-      best = ob;
-      best_j = oj;
+  for (int msk = 32; msk >= 1; msk >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, msk, 64));
+  if (lane == 0) wmax[wv] = top;
+  if (nan) s_fail = 1u;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) top = max(top, wmax[i]);
+  const float m = capped_x(top);
+
+  // ---- the block, then the index, that holds the K-th largest value --------------------------------
+  if (wv == 0) {  // lane l: block 63 - l, inclusive count from the top
+    const uint32_t mine = blk[63 - lane];
+    uint32_t cum = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t v = (uint32_t)__shfl_up((int)cum, d, 64);
+      if (lane >= d) cum += v;
+    }
+    const uint64_t hit = __ballot(cum >= (uint32_t)K);
+    if (lane == 63 && cum != (uint32_t)V) s_fail = 1u;  // a counter overflowed
+    if (lane == (hit ? __ffsll((long long)hit) - 1 : 63)) {
+      s_block = (uint32_t)(63 - lane);
+      s_above = cum - mine;
     }
   }
-  if (lane == 0) {
-    s_best[wv] = best;
-    s_best_j[wv] = best_j;
-  }
   __syncthreads();
-  if (tid == 0) {
-    float b = s_best[0];
-    int j = s_best_j[0];
-    for (int i = 1; i < (K + 63) / 64; ++i)
-      if (beats(s_best[i], s_best_j[i], b, j)) {
-        b = s_best[i];
-        j = s_best_j[i];
-      }
-    j = j < 0 ? 0 : (j >= K ? K - 1 : j);
-    a.token_out[row] = prop_id[j];
-    a.logp_out[row] = (prop_x[j] - full.m) - logf(full.s);
+  {
+    const uint32_t b = s_block, need = (uint32_t)K - s_above;
+    const int t = kSampleThreads - 1 - tid;  // from the block's top down
+    const uint32_t w = hist[t + kSampleThreads * (int)(b & 31u)];
+    uint32_t cum = b >= 32u ? w >> 16 : w & 0xffffu;
+    const uint32_t mine = cum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t v = (uint32_t)__shfl_up((int)cum, d, 64);
+      if (lane >= d) cum += v;
+    }
+    if (lane == 63) wcnt[wv] = cum;
+    __syncthreads();
+    for (int i = 0; i < wv; ++i) cum += wcnt[i];
+    if (cum >= need && cum - mine < need) s_index = (uint32_t)t + 1024u * b;
   }
+  // ---- log-softmax sum: one exp per distinct value, added in f64 -----------------------------------
+  double part = 0.0;
+  for (int i = 0; i < 32; ++i) {
+    const uint32_t c = hist[tid + kSampleThreads * i], o = (uint32_t)(tid + kSampleThreads * i);
+    if (c >> 16) part += (double)(c >> 16) * (double)expf(capped_x(o + 0x8000u) - m);
+    if (c & 0xffffu) part += (double)(c & 0xffffu) * (double)expf(capped_x(o) - m);
+  }
+#pragma unroll
+  for (int msk = 32; msk >= 1; msk >>= 1) part += __shfl_xor(part, msk, 64);
+  if (lane == 0) wsum[wv] = part;
+  __syncthreads();
+  double total = 0.0;
+  for (int i = 0; i < NW; ++i) total += wsum[i];
+  // the smallest index whose score ties with the K-th: thread t looks at the t-th below it
+  const uint32_t kth = s_index;
+  const uint32_t key_k = key_of(capped_x(kth));
+  const bool below = (uint32_t)tid < kth && key_of(capped_x(kth - 1u - (uint32_t)tid)) >= key_k;
+  const uint64_t out = __ballot(!below);
+  if (lane == 0) wmax[wv] = out ? (uint32_t)(64 * wv + __ffsll((long long)out) - 1) : 0xffffffffu;
+  __syncthreads();  // (also: the counts are read; the candidates reuse their LDS)
+  uint32_t ties = 0xffffffffu;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) ties = min(ties, wmax[i]);
+  if (s_fail || ties == 0xffffffffu) {  // uniform
+    if (tid == 0) a.token_out[row] = kTkRedo;
+    return;
+  }
+  const uint32_t floor_o = kth - ties;
+
+  // ---- second pass: every column at or above it ------------------------------------------------------
+  uint32_t* cand_key = hist;
+  int32_t* cand_id = reinterpret_cast<int32_t*>(hist + kTkCand);
+  float* cand_x = reinterpret_cast<float*>(hist + 2 * kTkCand);
+  each_chunk([&](int j, u32x4 r) {
+    uint32_t o[4];
+    bool any = false;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      o[q] = order2(r[q]);
+      any = any || (o[q] & 0xffffu) >= floor_o || (o[q] >> 16) >= floor_o;
+    }
+    if (any && j < nchunks) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t oe = e & 1 ? o[e >> 1] >> 16 : o[e >> 1] & 0xffffu;
+        if (oe >= floor_o) {
+          const uint32_t pos = atomicAdd(&s_count, 1u);
+          if (pos < (uint32_t)kTkCand) {
+            const float x = capped_x(oe);
+            cand_key[pos] = key_of(x);
+            cand_id[pos] = 8 * j + e;
+            cand_x[pos] = x;
+          }
+        }
+      }
+    }
+  });
+  __syncthreads();
+  const uint32_t n_cand = s_count;
+  if (n_cand > (uint32_t)kTkCand) {
+    if (tid == 0) a.token_out[row] = kTkRedo;
+    return;
+  }
+  tk_draw(a, row, cand_key, cand_id, cand_x, n_cand, m, (float)total, prop);
 }
 
 }  // namespace
@@ -677,7 +895,10 @@ extern "C" int g4_sample_top_k(const G4SampleTopKArgs* args, void* stream) {
   const bool vec = a.vocab % 8 == 0 && (a.row_stride * esize) % 16 == 0 && reinterpret_cast<uintptr_t>(a.logits) % 16 == 0;
   const dim3 grid(a.batch), block(kSampleThreads);
   if (a.dtype == G4_DTYPE_BF16) {
-    if (vec)
+    if (vec && a.vocab >= kTkHistVocab) {
+      hipLaunchKernelGGL(sample_top_k_hist_kernel, grid, block, 0, st, a);
+      hipLaunchKernelGGL((sample_top_k_kernel<true, true, true>), grid, block, 0, st, a);
+    } else if (vec)
       hipLaunchKernelGGL((sample_top_k_kernel<true, true>), grid, block, 0, st, a);
     else
       hipLaunchKernelGGL((sample_top_k_kernel<true, false>), grid, block, 0, st, a);
