@@ -5,20 +5,19 @@
 //
 // One persistent grid of two workgroups per CU. A workgroup owns all M <= 256 rows and walks its
 // vocab tiles of 128 columns (tile t, t + grid, ...). Per tile: the GEMM over K in stages of 32
-// (x 256 x 32 and embed 128 x 32 DMA'd into a 3-slot LDS ring, two stages in flight; the ring runs
-// on across tiles, so the next tile's first stages load during this tile's epilogue), then the
+// (x ROWS x 32 and embed 128 x 32 DMA'd into an LDS ring, LhShape; the ring runs on across tiles, so the next tile's first stages load during this tile's epilogue), then the
 // epilogue on the accumulators in registers: bf16 rounding, the soft-cap, the running max / sum of
 // the full-vocab log-softmax, Gumbel noise from JAX's threefry stream and the running argmax.
 // The epilogue is VALU work (the threefry rounds dominate); the GEMM is weight streaming and MFMA,
 // so the two workgroups of a CU overlap one's epilogue with the other's GEMM.
 //
-// Wave w owns rows [64 w, 64 w + 64) x the tile's 128 columns: MFMA v_mfma_f32_16x16x32_bf16 with
-// A = 16 embed rows (vocab columns), B = 16 x rows; lane (grp, col) accumulates
-// logits[64 w + 16 rb + col][16 cb + 4 grp + j]. The lane keeps one running state per row it holds
+// Wave (wr, wc) owns rows [64 wr, 64 wr + 64) x 16 CB of the tile's 128 columns: MFMA
+// v_mfma_f32_16x16x32_bf16 with A = 16 embed rows (vocab columns), B = 16 x rows; lane (grp, col)
+// accumulates logits[64 wr + 16 rb + col][16 (CB wc + cb) + 4 grp + j]. The lane keeps one running state per row it holds
 // (rb = 0..3) across the workgroup's tiles, visiting its columns in increasing order, so a strict
 // comparison keeps the first of equal scores. At the end the 4 lanes of a row merge (column order
-// decides ties) and the workgroup writes one state per row; a combine kernel merges the
-// workgroups' states in workgroup order, writes the token and its log-probability, and splits the
+// decides ties) and each wave writes one state per row; a combine kernel merges the
+// states in workgroup and column order, writes the token and its log-probability, and splits the
 // loop key.
 #include "g4_common.h"
 #include "g4_internal.h"
@@ -28,20 +27,34 @@ namespace {
 
 #include "g4_sample_common.h"  // threefry2x32, Gumbel noise
 
-constexpr int kLhRows = 256;  // rows per workgroup (all of them)
+constexpr int kLhRows = 256;  // rows at most
 constexpr int kLhCols = 128;  // vocab columns per tile
 constexpr int kLhKT = 32;     // K per stage (one MFMA)
-constexpr int kLhSlots = 3;   // LDS ring slots: two stages in flight
 constexpr int kLhThreads = 256;
-constexpr int kLhXBytes = kLhRows * kLhKT * 2;   // 16 KiB: 256 rows x 64 bytes
 constexpr int kLhWBytes = kLhCols * kLhKT * 2;   // 8 KiB: 128 rows x 64 bytes
-constexpr int kLhSlotBytes = kLhXBytes + kLhWBytes;
-constexpr int kLhDmaPerWave = (kLhRows + kLhCols) / 16 / 4;  // 16-row DMA groups per wave and stage: 6
 constexpr int kLhWgPerCu = 2;
+
+// A workgroup's rows: 64, 128 or 256, the smallest that holds the batch. Fewer rows leave LDS for more ring
+// slots (the embedding bytes in flight, not the rows, bound a small batch: two stages of 8 KiB of it per
+// workgroup at 256 rows, five at 64) and spend neither DMA nor MFMA time on padding rows; the four waves
+// divide the 128 columns instead (ROWS / 64 waves along the rows). V = 262144, K = 2048, us at 1 / 64 / 128
+// rows: logits only 244 / 277 / 305 -> 204 / 247 / 273, with the T = 1 draw 271 / 390 / 457 -> 232 / 259 /
+// 322 (1 row reads the embedding at 5.3 TB/s).
+template <int ROWS>
+struct LhShape {
+  static constexpr int WR = ROWS / 64;              // waves along the rows
+  static constexpr int WC = 4 / WR;                 // along the columns
+  static constexpr int CB = kLhCols / 16 / WC;      // 16-column blocks per wave
+  static constexpr int X_BYTES = ROWS * kLhKT * 2;  // 16 KiB at 256 rows
+  static constexpr int SLOT = X_BYTES + kLhWBytes;
+  static constexpr int SLOTS = ROWS == 256 ? 3 : ROWS == 128 ? 4 : 6;  // LDS ring: SLOTS - 1 stages in flight
+  static constexpr int DMA = (ROWS + kLhCols) / 16 / 4;                // 16-row DMA groups per wave and stage
+  static_assert((ROWS + kLhCols) % 64 == 0, "every wave issues the same DMA count");
+};
 
 int g_lh_grid[kMaxDevices];  // persistent grid size per device (2 x CUs), set by setup_lm_head
 
-// Per-workgroup row states in the workspace: [grid][256] of each field.
+// Row states in the workspace: [grid x WC][ROWS] of each field (grid x 256 of them at every ROWS).
 struct LhStates {
   float* m;
   float* s;
@@ -94,18 +107,19 @@ __device__ __forceinline__ LhState lh_shfl(const LhState& x, int mask) {
 // instruction: 64 lanes x 16 bytes landing at lane * 16). Within a group, row r's 16-byte piece p
 // sits at 16-byte slot 4 r + (p ^ ((r >> 1) & 3)), so the 8 rows of an operand read's phase fall on
 // 8 different 16-byte bank groups; lane l fetches the piece that belongs at slot l (row l / 4, the
-// row's four pieces from the same 64-byte segment). Groups 0..15 are x rows, 16..23 embed rows;
-// wave w moves groups w, w + 4, ..., w + 20. x rows >= M read beyond the resource: zeros.
+// row's four pieces from the same 64-byte segment). Groups 0 .. ROWS / 16 - 1 are x rows, then eight of
+// embed rows; wave w moves groups w, w + 4, .... x rows >= M read beyond the resource: zeros.
 __device__ __forceinline__ int lh_swz(int r) { return (r >> 1) & 3; }
 
+template <int ROWS>
 __device__ __forceinline__ void lh_dma(unsigned char* __restrict__ slot, __amdgpu_buffer_rsrc_t rx,
                                        __amdgpu_buffer_rsrc_t rw, int K, int k0, int n0, int w, int lane) {
   const int rl = lane >> 2, piece = (lane & 3) ^ lh_swz(lane >> 2);
 #pragma unroll
-  for (int i = 0; i < kLhDmaPerWave; ++i) {
+  for (int i = 0; i < LhShape<ROWS>::DMA; ++i) {
     const int g = w + 4 * i;
-    const bool is_x = g < kLhRows / 16;
-    const int row = is_x ? 16 * g + rl : n0 + 16 * (g - kLhRows / 16) + rl;
+    const bool is_x = g < ROWS / 16;
+    const int row = is_x ? 16 * g + rl : n0 + 16 * (g - ROWS / 16) + rl;
     const uint32_t off = (uint32_t)(row * K + k0 + 8 * piece) * 2u;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(is_x ? rx : rw,
                                              (__attribute__((address_space(3))) void*)(slot + g * 1024), 16, off, 0,
@@ -113,24 +127,28 @@ __device__ __forceinline__ void lh_dma(unsigned char* __restrict__ slot, __amdgp
   }
 }
 
-// One stage's MFMAs for wave w: 4 x-row blocks (B operands) x 8 embed-row blocks (A operands).
-__device__ __forceinline__ void lh_compute(uint32_t slot, floatx4 (&acc)[4][8], int w, int col, int grp) {
+// One stage's MFMAs for wave (wr, wc): 4 x-row blocks (B operands) x CB embed-row blocks (A operands).
+template <int ROWS>
+__device__ __forceinline__ void lh_compute(uint32_t slot, floatx4 (&acc)[4][LhShape<ROWS>::CB], int wr, int wc, int col,
+                                           int grp) {
+  constexpr int CB = LhShape<ROWS>::CB;
   // row 16 b + col of a part, piece grp: group b, slot 4 col + (grp ^ swz(col))
   const uint32_t in_group = (uint32_t)col * 64u + (uint32_t)(grp ^ lh_swz(col)) * 16u;
-  const uint32_t xs = slot + (uint32_t)(4 * w) * 1024u + in_group;
-  const uint32_t ws = slot + (uint32_t)kLhXBytes + in_group;
-  u32x4 b[4], a[8];
+  const uint32_t xs = slot + (uint32_t)(4 * wr) * 1024u + in_group;
+  const uint32_t ws = slot + (uint32_t)(LhShape<ROWS>::X_BYTES + wc * CB * 1024) + in_group;
+  u32x4 b[4], a[CB];
 #pragma unroll
-  for (int rb = 0; rb < 4; ++rb) b[rb] = lds_read16(xs + 1024u * rb);
+  for (int rb = 0; rb < 4; ++rb) b[rb] = lds_read16_at(xs, 1024 * rb);
 #pragma unroll
-  for (int cb = 0; cb < 8; ++cb) a[cb] = lds_read16(ws + 1024u * cb);
-  __asm__ volatile("s_waitcnt lgkmcnt(0)"
-                   : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]),
-                     "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]));
+  for (int cb = 0; cb < CB; ++cb) a[cb] = lds_read16_at(ws, 1024 * cb);
+#pragma unroll
+  for (int rb = 0; rb < 4; ++rb) lgkm_wait(0, b[rb]);
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) lgkm_wait(0, a[cb]);
 #pragma unroll
   for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-    for (int cb = 0; cb < 8; ++cb) acc[rb][cb] = mfma16x16x32(as_bf16x8(a[cb]), as_bf16x8(b[rb]), acc[rb][cb]);
+    for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mfma16x16x32(as_bf16x8(a[cb]), as_bf16x8(b[rb]), acc[rb][cb]);
 }
 
 // The epilogue of four consecutive columns n .. n + 3 of one row: bf16 rounding (the logits), the
@@ -182,13 +200,16 @@ __device__ __forceinline__ void lh_epilogue(floatx4 v, LhState& sr, int row, int
 
 // SAMPLE: run the sampler epilogue (else only the bf16 logits are written); GREEDY: no noise;
 // UNIT_T: temperature 1.
-template <bool SAMPLE, bool GREEDY, bool UNIT_T = false>
+template <int ROWS, bool SAMPLE, bool GREEDY, bool UNIT_T = false>
 __global__ __launch_bounds__(kLhThreads, kLhWgPerCu) void lm_head_kernel(G4LmHeadSampleArgs a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char ring[kLhSlots][kLhSlotBytes];
+  using S_ = LhShape<ROWS>;
+  constexpr int kLhSlots = S_::SLOTS;
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[kLhSlots][S_::SLOT];
   __shared__ uint16_t cap_tab[SAMPLE ? kCapTableEntries : 1];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
+  const int wr = w % S_::WR, wc = w / S_::WR;
   const int K = a.hidden, V = a.vocab, M = a.batch;
   const int nst = K / kLhKT;
   const int n_tiles = V / kLhCols;
@@ -217,49 +238,49 @@ __global__ __launch_bounds__(kLhThreads, kLhWgPerCu) void lm_head_kernel(G4LmHea
   }
 
   // the ring's stage sequence runs over every (tile, k stage) of this workgroup; stage q of the
-  // sequence sits in slot q % 3. Stages past the last tile re-read stage 0 of the last tile (an L2
+  // sequence sits in slot q % SLOTS. Stages past the last tile re-read stage 0 of the last tile (an L2
   // hit), so every wave issues the same number of DMAs per step.
   const int my_tiles = blockIdx.x < n_tiles ? (n_tiles - 1 - (int)blockIdx.x) / grid + 1 : 0;
   const int total = my_tiles * nst;
   auto issue = [&](int q) {
     const int qq = q < total ? q : (total > 0 ? total - nst : 0);
     const int t = (int)blockIdx.x + (qq / nst) * grid;
-    lh_dma(&ring[q % kLhSlots][0], rx, rw, K, (qq % nst) * kLhKT, t * kLhCols, w, lane);
+    lh_dma<ROWS>(&ring[q % kLhSlots][0], rx, rw, K, (qq % nst) * kLhKT, t * kLhCols, w, lane);
   };
   if (total > 0) {
-    issue(0);
-    issue(1);
+#pragma unroll
+    for (int i = 0; i < kLhSlots - 1; ++i) issue(i);
   }
   int q = 0;
   for (int it = 0; it < my_tiles; ++it) {
     const int n0 = ((int)blockIdx.x + it * grid) * kLhCols;
-    floatx4 acc[4][8];
+    floatx4 acc[4][S_::CB];
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-      for (int cb = 0; cb < 8; ++cb) acc[rb][cb] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int cb = 0; cb < S_::CB; ++cb) acc[rb][cb] = floatx4{0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < nst; ++s, ++q) {
-      // this wave's DMAs of stage q have landed (those of q + 1 may not have), then every wave's;
-      // every wave is also past stage q - 1, whose slot the DMAs of q + 2 refill
-      __asm__ volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kLhDmaPerWave) : "memory");
-      issue(q + 2);
-      lh_compute(ring0 + (uint32_t)(q % kLhSlots) * kLhSlotBytes, acc, w, col, grp);
+      // this wave's DMAs of stage q have landed (those of the stages behind it may not have), then every
+      // wave's; every wave is also past stage q - 1, whose slot the DMAs of q + SLOTS - 1 refill
+      __asm__ volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((kLhSlots - 2) * S_::DMA) : "memory");
+      issue(q + kLhSlots - 1);
+      lh_compute<ROWS>(ring0 + (uint32_t)(q % kLhSlots) * S_::SLOT, acc, wr, wc, col, grp);
     }
 
-    // ---- epilogue: lane (grp, col) holds logits[64 w + 16 rb + col][n0 + 16 cb + 4 grp + j] ----------
+    // ---- epilogue: lane (grp, col) holds logits[64 wr + 16 rb + col][n0 + 16 (CB wc + cb) + 4 grp + j] --
     // The cb loop stays a loop (code size): each iteration takes block acc[rb][0] and rotates the
-    // row's eight blocks by one, so every register index is static.
+    // row's CB blocks by one, so every register index is static.
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
-      const int row = 64 * w + 16 * rb + col;
+      const int row = 64 * wr + 16 * rb + col;
       if (row < M) {
 #pragma unroll 1
-        for (int cb = 0; cb < 8; ++cb) {
+        for (int cb = 0; cb < S_::CB; ++cb) {
           const floatx4 v = acc[rb][0];
 #pragma unroll
-          for (int i = 0; i < 7; ++i) acc[rb][i] = acc[rb][i + 1];
-          acc[rb][7] = v;
-          lh_epilogue<SAMPLE, GREEDY, UNIT_T>(v, st[rb], row, n0 + 16 * cb + 4 * grp, a, ct, k0, k1);
+          for (int i = 0; i + 1 < S_::CB; ++i) acc[rb][i] = acc[rb][i + 1];
+          acc[rb][S_::CB - 1] = v;
+          lh_epilogue<SAMPLE, GREEDY, UNIT_T>(v, st[rb], row, n0 + 16 * (S_::CB * wc + cb) + 4 * grp, a, ct, k0, k1);
         }
       }
     }
@@ -267,16 +288,16 @@ __global__ __launch_bounds__(kLhThreads, kLhWgPerCu) void lm_head_kernel(G4LmHea
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the trailing DMAs land before the wave ends
 
   if constexpr (SAMPLE) {
-    // the 4 lanes of a row (grp 0..3) merge; lane grp = 0 writes the workgroup's state of the row
+    // the 4 lanes of a row (grp 0..3) merge; lane grp = 0 writes the wave's state of the row
     const LhStates ws = lh_states(a.workspace, grid);
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
       LhState x = st[rb];
       lh_merge(x, lh_shfl(x, 16));
       lh_merge(x, lh_shfl(x, 32));
-      const int row = 64 * w + 16 * rb + col;
+      const int row = 64 * wr + 16 * rb + col;
       if (grp == 0 && row < M) {
-        const size_t i = (size_t)blockIdx.x * kLhRows + row;
+        const size_t i = ((size_t)blockIdx.x * S_::WC + wc) * ROWS + row;
         ws.m[i] = x.m;
         ws.s[i] = x.s;
         ws.best[i] = x.best;
@@ -292,7 +313,8 @@ __global__ __launch_bounds__(kLhThreads, kLhWgPerCu) void lm_head_kernel(G4LmHea
 // 0 then splits the loop key (every workgroup of the LM head kernel has read it).
 constexpr int kCombineThreads = 256;
 
-__global__ __launch_bounds__(kCombineThreads) void lm_head_combine_kernel(G4LmHeadSampleArgs a, int grid) {
+__global__ __launch_bounds__(kCombineThreads) void lm_head_combine_kernel(G4LmHeadSampleArgs a, int grid,
+                                                                               int rows) {
   __shared__ LhState red[kCombineThreads];
   // Workgroups are dealt to the 8 XCDs round robin (blockIdx mod 8). The states of consecutive rows
   // share cache lines (32 rows per 128-byte line of each array), so each XCD takes a contiguous
@@ -300,22 +322,23 @@ __global__ __launch_bounds__(kCombineThreads) void lm_head_combine_kernel(G4LmHe
   const int wg = (int)blockIdx.x;
   const int row = a.batch % 8 == 0 ? (wg & 7) * (a.batch >> 3) + (wg >> 3) : wg;
   const LhStates ws = lh_states(a.workspace, grid);
+  const int n_states = grid * (kLhRows / rows);
   LhState st = {kF32Min, 0.f, -INFINITY, 0.f, 0x7fffffff};
   // states g = tid, tid + 256, ... merged in that order; two of them are requested before either
   // is merged (one round trip for the 512-workgroup grid of 256 CUs)
-  for (int g0 = threadIdx.x; g0 < grid; g0 += 2 * kCombineThreads) {
+  for (int g0 = threadIdx.x; g0 < n_states; g0 += 2 * kCombineThreads) {
     LhState v[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int g = g0 + u * kCombineThreads;
-      if (g < grid) {
-        const size_t i = (size_t)g * kLhRows + row;
+      if (g < n_states) {
+        const size_t i = (size_t)g * rows + row;
         v[u] = LhState{ws.m[i], ws.s[i], ws.best[i], ws.bx[i], ws.idx[i]};
       }
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u)
-      if (g0 + u * kCombineThreads < grid) lh_merge(st, v[u]);
+      if (g0 + u * kCombineThreads < n_states) lh_merge(st, v[u]);
   }
   // tree: at level h thread t < h merges thread t + h (h = 128, 64 through LDS, then 32 .. 1 by
   // shuffles within wave 0, where lane t reads lane t ^ h = t + h)
@@ -348,6 +371,19 @@ __global__ __launch_bounds__(kCombineThreads) void lm_head_combine_kernel(G4LmHe
       a.key[1] = x1;
     }
   }
+}
+
+template <int ROWS>
+void launch_lm_head(const G4LmHeadSampleArgs& a, int grid, hipStream_t st) {
+  const dim3 g((unsigned)grid), b(kLhThreads);
+  if (!a.token_out)
+    hipLaunchKernelGGL((lm_head_kernel<ROWS, false, true>), g, b, 0, st, a);
+  else if (!(a.temperature > 0.f))
+    hipLaunchKernelGGL((lm_head_kernel<ROWS, true, true>), g, b, 0, st, a);
+  else if (a.temperature == 1.0f)
+    hipLaunchKernelGGL((lm_head_kernel<ROWS, true, false, true>), g, b, 0, st, a);
+  else
+    hipLaunchKernelGGL((lm_head_kernel<ROWS, true, false>), g, b, 0, st, a);
 }
 
 int lh_grid(const G4LmHeadSampleArgs& a, int dev) {
@@ -418,16 +454,15 @@ extern "C" int g4_lm_head_sample(const G4LmHeadSampleArgs* args, void* stream) {
       return fail(G4_ERR_INVALID, "g4_lm_head_sample: workspace needs 4-byte alignment");
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (!sample)
-    hipLaunchKernelGGL((lm_head_kernel<false, true>), dim3((unsigned)grid), dim3(kLhThreads), 0, st, a);
-  else if (greedy)
-    hipLaunchKernelGGL((lm_head_kernel<true, true>), dim3((unsigned)grid), dim3(kLhThreads), 0, st, a);
-  else if (a.temperature == 1.0f)
-    hipLaunchKernelGGL((lm_head_kernel<true, false, true>), dim3((unsigned)grid), dim3(kLhThreads), 0, st, a);
+  const int rows = a.batch <= 64 ? 64 : a.batch <= 128 ? 128 : 256;
+  if (rows == 64)
+    launch_lm_head<64>(a, grid, st);
+  else if (rows == 128)
+    launch_lm_head<128>(a, grid, st);
   else
-    hipLaunchKernelGGL((lm_head_kernel<true, false>), dim3((unsigned)grid), dim3(kLhThreads), 0, st, a);
+    launch_lm_head<256>(a, grid, st);
   if (int rc = check_launch("g4_lm_head_sample")) return rc;
   if (!sample) return G4_OK;
-  hipLaunchKernelGGL(lm_head_combine_kernel, dim3((unsigned)a.batch), dim3(kCombineThreads), 0, st, a, grid);
+  hipLaunchKernelGGL(lm_head_combine_kernel, dim3((unsigned)a.batch), dim3(kCombineThreads), 0, st, a, grid, rows);
   return check_launch("g4_lm_head_sample (combine)");
 }

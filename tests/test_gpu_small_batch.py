@@ -93,3 +93,27 @@ def test_few_row_linear(device, rows, n, k):
     # g and u one rounding apart at most (2^-8 relative each, gelu'(g) <= 1.13 and gelu(g) ~ g / 2 below)
     bar = 2.0 ** -7 * (want.abs() + 1.2 * gate.abs() * up.abs()) + 2.0 * slack.chunk(2, -1)[0] * up.abs() + 1e-6
     assert torch.all((got - want).abs() <= bar)
+
+
+# the last batch of each row shape (64, 128, 256 rows per workgroup) and the first of the next
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 128, 129])
+@pytest.mark.parametrize("vocab,hidden", [(128, 32), (1280, 96)])
+def test_lm_head_row_shapes(device, rows, vocab, hidden):
+    """Logits within the bf16 rounding of their f32 sums; the draw on them equals sample_tokens' on the
+    stored logits, token for token, at T = 1, another temperature and greedy (logp: f32 sums in another
+    order, the reference's 2e-6)."""
+
+    g = torch.Generator(device="cuda").manual_seed(rows + vocab)
+    x = torch.randn((rows, hidden), device="cuda", generator=g).to(torch.bfloat16)
+    embed = (torch.randn((vocab, hidden), device="cuda", generator=g) * 0.5).to(torch.bfloat16)
+    logits = kernels.lm_head(x, embed)
+    ref = x.double() @ embed.double().T
+    slack = 2.0 ** -20 * (x.double().abs() @ embed.double().abs().T)
+    assert torch.all((logits.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + slack)
+    key = torch.tensor([5, 6], dtype=torch.int32, device=device)
+    for temperature in (1.0, 0.6, 0.0):
+        args = dict(softcap=30.0, temperature=temperature, key=key, split_key=False)
+        tok, logp = kernels.lm_head_sample(x, embed, **args)
+        want_tok, want_logp = kernels.sample_tokens(logits, **args)
+        assert torch.equal(tok, want_tok)
+        assert torch.all((logp - want_logp).abs() <= 2e-6)
