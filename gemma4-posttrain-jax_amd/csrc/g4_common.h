@@ -83,15 +83,52 @@ template <> struct Elem<false> {
   __device__ static __forceinline__ float round(float v) { return v; }
 };
 
-// Wave64 reductions over lanes that differ in the given xor masks.
-__device__ __forceinline__ float wave_sum(float v) {
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  return v;
+// A lane's value moved by a DPP control word (every lane active, every source lane within its row).
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  const int u = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(u, u, CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float wave_max(float v) {
-  for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-  return v;
+
+// Wave64 reductions, the result in every lane.
+// Each step reads its partner by a lane permutation in the vector pipeline (v_permlane32/16_swap_b32,
+// then DPP), not by ds_bpermute through LDS (__shfl_xor): the six steps are one dependent chain.
+// Once the masks 32, 16 and 8 are done a value repeats every 8 lanes of its row, so that a row
+// rotation by 4 reads lane ^ 4's value; every step combines the same two values as the xor butterfly
+// from 32 down to 1, so the result has the same bits. Every lane of the wave has to be active.
+// Twelve 512-slot decode layers of one row 117 -> 111 us, the E2B-like step at 256 rows 4.41 -> 4.31 ms,
+// the append of 256 x 256 tokens 371 -> 354 us.
+template <typename F>
+__device__ __forceinline__ float across32(float v, F op) {  // op(v, v of lane ^ 32), commutative
+  const uint32_t u = __float_as_uint(v);
+  const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // lanes l % 32 and l % 32 + 32
+  return op(__uint_as_float(s[0]), __uint_as_float(s[1]));
 }
+template <typename F>
+__device__ __forceinline__ float across16(float v, F op) {  // op(v, v of lane ^ 16), commutative
+  const uint32_t u = __float_as_uint(v);
+  const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // the even / odd row of 16 lanes
+  return op(__uint_as_float(s[0]), __uint_as_float(s[1]));
+}
+template <typename F>
+__device__ __forceinline__ float wave_reduce(float v, F op) {
+  v = across16(across32(v, op), op);
+  v = op(v, dpp<0x128>(v));    // row_ror:8
+  v = op(v, dpp<0x124>(v));    // row_ror:4
+  v = op(v, dpp<0x4e>(v));     // quad_perm:[2,3,0,1]
+  return op(v, dpp<0xb1>(v));  // quad_perm:[1,0,3,2]
+}
+struct SumOp {
+  __device__ __forceinline__ float operator()(float x, float y) const { return x + y; }
+};
+struct MaxOp {
+  __device__ __forceinline__ float operator()(float x, float y) const { return fmaxf(x, y); }
+};
+__device__ __forceinline__ float wave_sum(float v) { return wave_reduce(v, SumOp()); }
+__device__ __forceinline__ float wave_max(float v) { return wave_reduce(v, MaxOp()); }
+// over the four lanes that share l % 16 (the row groups of one MFMA column)
+__device__ __forceinline__ float column_sum(float v) { return across32(across16(v, SumOp()), SumOp()); }
+__device__ __forceinline__ float column_max(float v) { return across32(across16(v, MaxOp()), MaxOp()); }
 
 // Ring slot r of a Wc-slot buffer holds the greatest position p <= last with p % Wc == r
 // (model.py:357); negative means never written.

@@ -183,8 +183,7 @@ struct Softmax {
 // Row max and sum over every scanned slot (two LDS rounds across the waves).
 __device__ __forceinline__ Softmax softmax_stats(float mx, const float* sc, float* wmax, float* wsum, int t_alloc,
                                                  int n_chunks, int R, int w, int col, int grp) {
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = column_max(mx);
   if (grp == 0) wmax[w * 16 + col] = mx;
   __syncthreads();
   Softmax sm;
@@ -204,8 +203,7 @@ __device__ __forceinline__ Softmax softmax_stats(float mx, const float* sc, floa
       for (int e = 0; e < 8; ++e) l += expf(sp[e] - sm.m);
     }
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = column_sum(l);
   if (grp == 0) wsum[w * 16 + col] = l;
   __syncthreads();
   sm.l = 0.f;

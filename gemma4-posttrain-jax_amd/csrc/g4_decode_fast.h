@@ -316,8 +316,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void decode_bf16_fast_kernel(G4D
   }
 
   // ---- 4. softmax statistics and probabilities --------------------------------------------------
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = column_max(mx);
   if (grp == 0) L.wmax[w * 16 + col] = mx;
   __syncthreads();
   float m = kBf16Min;
@@ -335,8 +334,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64) void decode_bf16_fast_kernel(G4D
       for (int q = 0; q < 4; ++q) l += expf(bf16_lo(sv[q]) - m) + expf(bf16_hi(sv[q]) - m);
     }
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = column_sum(l);
   if (grp == 0) L.wsum[w * 16 + col] = l;
   __syncthreads();
   float lt = 0.f;

@@ -131,8 +131,7 @@ decode_bf16_splitk_scores_kernel(G4DecodeArgs a,
     patch_k_sel<D>(kc1, nk_lds, kr.new_slot, c1, col, grp);
     mx = score(kc1, vb1, 32 * (w + NW), mx);
   }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = column_max(mx);
   if (grp == 0) wmax[w * 16 + col] = mx;
   __syncthreads();
 
@@ -152,7 +151,7 @@ decode_bf16_splitk_scores_kernel(G4DecodeArgs a,
       float part = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) part += slot + j < n_local ? expf(s4[j] - msplit[i]) : 0.f;
-      part = wave_sum64(part);
+      part = wave_sum(part);
       if (lane == 0) bsum[2 * hh + (w & 1)] = part;
       // the split's scores to the workspace (slots beyond n_local are never read)
       *reinterpret_cast<uint2*>(ws.scores + ((int64_t)pair * R + hh) * ws.c_pad + split * kSplitSlots + slot) = sv;
@@ -196,15 +195,14 @@ __device__ __forceinline__ bool splitk_row_stats(const SplitKWorkspace& ws, int 
 #pragma unroll
     for (int j = 0; j < 4; ++j) m = fmaxf(m, v[j].x);
     for (int s = lane + 256; s < n_splits_row; s += 64) m = fmaxf(m, st[(s * R + hh) * 2]);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    m = wave_max(m);
     // l = sum_s l_s * exp(m_s - m), per lane in split order, then across lanes in a fixed tree
     float l = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (lane + 64 * j < n_splits_row) l += v[j].y * expf(v[j].x - m);
     for (int s = lane + 256; s < n_splits_row; s += 64) l += st[(s * R + hh) * 2 + 1] * expf(st[(s * R + hh) * 2] - m);
-    l = wave_sum64(l);
+    l = wave_sum(l);
     if (lane == 0) {
       mh[hh] = m;
       lh[hh] = l;

@@ -30,12 +30,6 @@ constexpr int kStageSlots = 2 * NW * 32;  // slots per row handled here (16 chun
 // 0..3 on different banks for the 16-byte MFMA-operand accesses (lane (grp, col) -> row col).
 constexpr int kStageStride = kStageSlots + 32;
 
-__device__ __forceinline__ float wave_sum64(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
 constexpr int kVtEarly = 11;                // V^T chunks requested with K (the rest after the softmax)
 constexpr int kVtLate = 2 * NW - kVtEarly;
 template <int N>
@@ -134,8 +128,7 @@ __device__ __forceinline__ void stage_body(const G4DecodeArgs& a, VtTiles<kVtEar
     patch_k_sel<D>(k1, nk_lds, kr.new_slot, c1, col, grp);
     mx = score_to_lds<D>(k1, qop, vb1, sp, kStageStride, c1, R, col, grp, mx);
   }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = column_max(mx);
   if (grp == 0) wmax[w * 16 + col] = mx;
   wg_barrier();  // scores and wave maxima are in LDS
 
@@ -162,7 +155,7 @@ __device__ __forceinline__ void stage_body(const G4DecodeArgs& a, VtTiles<kVtEar
         ev[i][j] = slot + j < n_scanned ? expf(s4[j] - m) : 0.f;
         part += ev[i][j];
       }
-      part = wave_sum64(part);
+      part = wave_sum(part);
       if (lane == 0) bsum[2 * hh + (w & 1)] = part;
     }
   }
