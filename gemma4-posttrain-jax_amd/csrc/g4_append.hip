@@ -120,124 +120,244 @@ __global__ __launch_bounds__(1024) void append_kernel(G4AppendArgs a) {
   }
 }
 
-// Prefill-sized appends (bf16, the vectorized rows, S >= 8): one 8-wave workgroup per 8
-// consecutive tokens of a row, one head vector per wave at a time, at 8 waves per SIMD (the
-// prepared vector and its loads take under 64 registers; D = 512 runs at 4). The value cache groups
-// 8 slots per 16-byte piece (cache_vt[b, h, slot / 8, d, slot % 8]), so one token's V row is D
-// two-byte pieces spread over D / 8 cache lines; when the 8 tokens land in one aligned 8-slot group
-// (a cache start and ring size that are multiples of 8) their V rows are staged in LDS and stored as
-// whole 16-byte pieces, 16 D contiguous bytes per head, and the chunk copy (vt_out) likewise. Other
-// workgroups store V element by element as append_kernel does. Same arithmetic and destinations as
-// append_kernel (E2B prefill shape, B 256 x S 256, D 256: a ring layer with its chunk copy 657 -> 421
-// us, a linear layer 494 -> 353 us, q alone 251 -> 232 us).
+// Prefill-sized appends (bf16, the vectorized rows, S >= 8): one 8-wave workgroup per 8 consecutive
+// tokens of a row, one token per wave. A token's cos / sin row and the norm weights are read and
+// rounded once for its H (R + 2) head vectors, whose loads are issued kTileVecs at a time (8 waves
+// per SIMD; D = 512 runs at 4). The value cache groups 8 slots per 16-byte piece
+// (cache_vt[b, h, slot / 8, d, slot % 8]), so one token's V row is D two-byte pieces spread over
+// D / 8 cache lines; when the 8 tokens land in one aligned 8-slot group (a cache start and ring size
+// that are multiples of 8) their V rows are staged in LDS and stored as whole 16-byte pieces, 16 D
+// contiguous bytes per head, and the chunk copy (vt_out) likewise. Other workgroups store V element
+// by element as append_kernel does. Same arithmetic and destinations as append_kernel.
+// Bound by HBM: 256 x 256 tokens of 2 x (4 + 2) heads of 256 with the chunk copy move 1.07 GB in 202 - 209
+// us, 5.2 TB/s (a copy of 4 GiB reaches 4.8); with a wave per head vector, which read the cos / sin row and
+// formed the slot anew for each of the 12 vectors of a token and rotated through LDS, 354 us.
 constexpr int kTileTok = 8;
-constexpr int kTileThreads = 512;
+constexpr int kTileThreads = 64 * kTileTok;
 constexpr int kTileVtBytes = 32 * 1024;  // LDS for the staged V rows: kv_heads * D * 16 bytes at most
+constexpr int kTileVecs = 4;             // head vectors of a token in flight per wave
+
+__device__ __forceinline__ void swap_halves(float& x, float& y) {  // x's lanes 32 .. 63 <-> y's lanes 0 .. 31
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  x = __uint_as_float(r[0]);
+  y = __uint_as_float(r[1]);
+}
+
+// The lane's PER elements as packed bf16 pairs, one access (PER = 2, 4 or 8).
+template <int W>
+__device__ __forceinline__ void ld_words(const uint16_t* p, uint32_t (&w)[W]) {
+  if constexpr (W == 1) {
+    w[0] = *reinterpret_cast<const uint32_t*>(p);
+  } else if constexpr (W == 2) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    w[0] = v.x, w[1] = v.y;
+  } else {
+    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = v[i];
+  }
+}
+template <int W>
+__device__ __forceinline__ void st_words(uint16_t* p, const uint32_t (&w)[W]) {
+  if constexpr (W == 1) {
+    *reinterpret_cast<uint32_t*>(p) = w[0];
+  } else if constexpr (W == 2) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(w[0], w[1]);
+  } else {
+    *reinterpret_cast<u32x4*>(p) = u32x4{w[0], w[1], w[2], w[3]};
+  }
+}
+
+// One token's RoPE row, rounded to bf16. Element pair (e, e + PER / 2) of a lane after swap_halves:
+// lanes 0 .. 31 hold dims d and d + D / 2 of element e, lanes 32 .. 63 those of element e + PER / 2,
+// so both members of a rotated pair sit in one lane and no partner is fetched.
+template <int PER>
+struct TileRope {
+  float c[PER], s[PER];
+  __device__ __forceinline__ void load(const float* rcos, const float* rsin, int lane) {
+    ld_f32<PER>(rcos + lane * PER, c);
+    ld_f32<PER>(rsin + lane * PER, s);
+  }
+  __device__ __forceinline__ void arrange() {
+#pragma unroll
+    for (int e = 0; e < PER / 2; ++e) {
+      swap_halves(c[e], c[e + PER / 2]);
+      swap_halves(s[e], s[e + PER / 2]);
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) c[e] = round_bf16(c[e]), s[e] = round_bf16(s[e]);
+  }
+};
+
+// prep_math on packed pairs: the same operations in the same order, so the same bits.
+template <int D, bool HAS_W>
+__device__ __forceinline__ void tile_prep(uint32_t (&w)[D / 128], bool norm, const float (&wv)[D / 64], bool rope,
+                                          const TileRope<D / 64>& tr, float eps) {
+#pragma clang fp contract(off)
+  constexpr int PER = D / 64, W = D / 128;
+  float x[PER];
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    x[2 * i] = __uint_as_float(w[i] << 16);
+    x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+  }
+  if (norm) {
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) ss += x[e] * x[e];
+    ss = wave_sum(ss);
+    const float inv = 1.0f / __fsqrt_rn(ss / (float)D + eps);
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      x[e] = x[e] * inv;
+      if (HAS_W) x[e] = x[e] * wv[e];
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i) w[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);
+  }
+  if (rope) {
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      x[2 * i] = __uint_as_float(w[i] << 16);
+      x[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+#pragma unroll
+    for (int e = 0; e < PER / 2; ++e) {
+      float lo = x[e], hi = x[e + PER / 2];
+      swap_halves(lo, hi);
+      const float lc = lo * tr.c[e], hs = -hi * tr.s[e];
+      const float hc = hi * tr.c[e + PER / 2], ls = lo * tr.s[e + PER / 2];
+      lo = lc + hs;
+      hi = hc + ls;
+      swap_halves(lo, hi);
+      x[e] = lo;
+      x[e + PER / 2] = hi;
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i) w[i] = pack_bf16x2(x[2 * i], x[2 * i + 1]);
+  }
+}
 
 template <int D>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(D >= 512 ? 4 : 8))) void
 append_tile_kernel(G4AppendArgs a) {
   using T = uint16_t;
-  constexpr int PER = D / 64;
-  extern __shared__ __attribute__((aligned(16))) uint16_t vt_lds[];  // [H][D][8]
+  constexpr int PER = D / 64, W = D / 128;
+  extern __shared__ __attribute__((aligned(16))) uint16_t v_lds[];  // [H][8 tokens][D]
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int nwaves = blockDim.x >> 6;
-  const int S = a.seq, H = a.kv_heads, R = a.group;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int S = a.seq, H = a.kv_heads;
   const int ntile = (S + kTileTok - 1) / kTileTok;
   const int b = (int)blockIdx.x / ntile;
   const int s0 = ((int)blockIdx.x - b * ntile) * kTileTok;
   const int n_tok = S - s0 < kTileTok ? S - s0 : kTileTok;
-  const int nq = a.q ? H * R : 0;
-  const int nvec = nq + (a.k ? 2 * H : 0);
 
-  // destination slot of token s (model.py:373-390), as in append_kernel
+  // destination slot of token s0 + t (model.py:373-390), as in append_kernel
   const int64_t start = a.write_pos ? (int64_t)a.write_pos[b] : (int64_t)a.write_pos_scalar;
-  const int64_t cap = a.capacity;
-  auto slot_of = [&](int s, bool& to_cache) -> int64_t {
-    if (a.kind == G4_CACHE_RING) {
-      const int64_t keep = S < cap ? S : cap;
-      to_cache = s >= S - keep;
-      return floor_mod(start + s, cap);
-    }
-    int64_t st = start < 0 ? 0 : start;
-    if (st > cap - S) st = cap - S;
-    to_cache = true;
-    return st + s;
+  const int cap = a.capacity;
+  const bool ring = a.kind == G4_CACHE_RING;
+  const int drop = ring && S > cap ? S - cap : 0;  // a ring keeps the chunk's last `cap` tokens
+  int64_t first = start < 0 ? 0 : start;
+  if (ring) {
+    first = floor_mod(start + s0, (int64_t)cap);
+  } else {
+    if (first > cap - S) first = cap - S;
+    first += s0;
+  }
+  auto slot_of = [&](int t) -> int64_t {
+    return ring ? (int64_t)(((uint32_t)first + (uint32_t)t) % (uint32_t)cap) : first + t;
   };
-  bool tc_first, tc_last;
-  const int64_t slot_first = slot_of(s0, tc_first);
-  const int64_t slot_last = slot_of(s0 + n_tok - 1, tc_last);
-  // whole 8-slot groups: 8 tokens, consecutive slots from a multiple of 8, one to_cache value
-  // (it only switches from false to true along the chunk)
-  const bool grouped = a.k && n_tok == kTileTok && slot_first % 8 == 0 && slot_last == slot_first + 7 &&
-                       tc_first == tc_last;
+  // whole 8-slot groups: 8 tokens, consecutive slots from a multiple of 8, all or none of them kept
+  const bool grouped = a.k && n_tok == kTileTok && first % 8 == 0 && slot_of(kTileTok - 1) == first + kTileTok - 1 &&
+                       (s0 >= drop) == (s0 + kTileTok - 1 >= drop);
 
-  const int jobs = n_tok * nvec;  // job = (token, head vector), tokens outermost
-  for (int job = wave; job < jobs; job += nwaves) {
-    const int t = job / nvec, vec = job - t * nvec;
-    const int s = s0 + t;
-    const int64_t in_base = ((int64_t)b * S + s) * a.in_row_stride;
-    int kind, head, r = 0;
-    const T* src;
-    if (vec < nq) {
-      kind = kQ;
-      head = vec / R;
-      r = vec - head * R;
-      src = reinterpret_cast<const T*>(a.q) + in_base + (int64_t)vec * D;
-    } else if (vec < nq + H) {
-      kind = kK;
-      head = vec - nq;
-      src = reinterpret_cast<const T*>(a.k) + in_base + (int64_t)head * D;
-    } else {
-      kind = kV;
-      head = vec - nq - H;
-      src = reinterpret_cast<const T*>(a.v) + in_base + (int64_t)head * D;
-    }
-    const bool norm = (kind == kQ && (a.flags & G4_APPEND_NORM_Q)) || (kind == kK && (a.flags & G4_APPEND_NORM_K)) ||
-                      (kind == kV && (a.flags & G4_APPEND_NORM_V));
-    const bool rope = (kind == kQ && (a.flags & G4_APPEND_ROPE_Q)) || (kind == kK && (a.flags & G4_APPEND_ROPE_K));
-    const T* w = norm ? (kind == kQ ? reinterpret_cast<const T*>(a.q_norm_weight)
-                                    : (kind == kK ? reinterpret_cast<const T*>(a.k_norm_weight) : nullptr))
-                      : nullptr;
-    const int64_t rope_base = ((int64_t)b * S + s) * D;
-    float x[PER];
-    prep_head<true, D, true>(src, w, norm, rope, a.rope_cos + rope_base, a.rope_sin + rope_base, a.eps, lane, x);
-    const int64_t bh = (int64_t)b * H + head;
-    if (kind == kQ) {
-      st_bf16<PER>(reinterpret_cast<T*>(a.q_out) + ((((int64_t)b * S + s) * H + head) * R + r) * D + lane * PER, x);
-      continue;
-    }
-    bool to_cache;
-    const int64_t slot = slot_of(s, to_cache);
-    if (kind == kK) {
-      if (to_cache) st_bf16<PER>(reinterpret_cast<T*>(a.cache_k) + bh * a.slot_stride * D + kt_index(slot, lane * PER, D), x);
-      if (a.k_out) st_bf16<PER>(reinterpret_cast<T*>(a.k_out) + bh * a.chunk_stride * D + kt_index(s, lane * PER, D), x);
-    } else if (grouped) {
+  if (wave < n_tok) {
+    const int t = wave, s = s0 + t;
+    const int64_t token = (int64_t)b * S + s;
+    const int64_t in_off = token * a.in_row_stride + lane * PER;
+    const bool rope_q = a.q && (a.flags & G4_APPEND_ROPE_Q), rope_k = a.k && (a.flags & G4_APPEND_ROPE_K);
+    TileRope<PER> tr;
+    if (rope_q || rope_k) tr.load(a.rope_cos + token * D, a.rope_sin + token * D, lane);
+    uint32_t w[kTileVecs][W];
+    float wv[PER];
+    bool arranged = false;
+    if (a.q) {
+      const bool norm = a.flags & G4_APPEND_NORM_Q;
+      const int nq = H * a.group;
+      const T* src = reinterpret_cast<const T*>(a.q) + in_off;
+      T* dst = reinterpret_cast<T*>(a.q_out) + token * nq * D + lane * PER;
+      if (norm) ld_bf16<PER>(reinterpret_cast<const T*>(a.q_norm_weight) + lane * PER, wv);
+      for (int v0 = 0; v0 < nq; v0 += kTileVecs) {
 #pragma unroll
-      for (int e = 0; e < PER; ++e) vt_lds[((int64_t)head * D + lane * PER + e) * 8 + t] = (uint16_t)f32_to_bf16_bits(x[e]);
-    } else {
-      if (to_cache) {
-        T* dst = reinterpret_cast<T*>(a.cache_vt) + bh * D * a.slot_stride;
+        for (int i = 0; i < kTileVecs; ++i)
+          if (v0 + i < nq) ld_words<W>(src + (v0 + i) * D, w[i]);
+        if (!arranged && (rope_q || rope_k)) tr.arrange();
+        arranged = true;
 #pragma unroll
-        for (int e = 0; e < PER; ++e) dst[vt_index(slot, lane * PER + e, D)] = (uint16_t)f32_to_bf16_bits(x[e]);
+        for (int i = 0; i < kTileVecs; ++i) {
+          if (v0 + i < nq) {
+            tile_prep<D, true>(w[i], norm, wv, rope_q, tr, a.eps);
+            st_words<W>(dst + (v0 + i) * D, w[i]);
+          }
+        }
       }
-      if (a.vt_out) {
-        T* dst = reinterpret_cast<T*>(a.vt_out) + bh * D * a.chunk_stride;
+    }
+    if (a.k) {
+      const bool norm_k = a.flags & G4_APPEND_NORM_K, norm_v = a.flags & G4_APPEND_NORM_V;
+      const T* ksrc = reinterpret_cast<const T*>(a.k) + in_off;
+      const T* vsrc = reinterpret_cast<const T*>(a.v) + in_off;
+      const bool to_cache = s >= drop;
+      const int64_t slot = slot_of(t);
+      const int64_t k_lane = kt_index(0, lane * PER, D);
+      if (norm_k) ld_bf16<PER>(reinterpret_cast<const T*>(a.k_norm_weight) + lane * PER, wv);
+      for (int h0 = 0; h0 < H; h0 += kTileVecs / 2) {
 #pragma unroll
-        for (int e = 0; e < PER; ++e) dst[vt_index(s, lane * PER + e, D)] = (uint16_t)f32_to_bf16_bits(x[e]);
+        for (int i = 0; i < kTileVecs / 2; ++i) {
+          if (h0 + i < H) {
+            ld_words<W>(ksrc + (h0 + i) * D, w[2 * i]);
+            ld_words<W>(vsrc + (h0 + i) * D, w[2 * i + 1]);
+          }
+        }
+        if (!arranged && rope_k) tr.arrange();
+        arranged = true;
+#pragma unroll
+        for (int i = 0; i < kTileVecs / 2; ++i) {
+          const int head = h0 + i;
+          if (head >= H) break;
+          const int64_t bh = (int64_t)b * H + head;
+          tile_prep<D, true>(w[2 * i], norm_k, wv, rope_k, tr, a.eps);
+          if (to_cache)
+            st_words<W>(reinterpret_cast<T*>(a.cache_k) + bh * a.slot_stride * D + kt_index(slot, 0, D) + k_lane, w[2 * i]);
+          if (a.k_out)
+            st_words<W>(reinterpret_cast<T*>(a.k_out) + bh * a.chunk_stride * D + kt_index(s, 0, D) + k_lane, w[2 * i]);
+          uint32_t(&vw)[W] = w[2 * i + 1];
+          tile_prep<D, false>(vw, norm_v, wv, false, tr, a.eps);
+          if (grouped) {
+            st_words<W>(v_lds + (head * kTileTok + t) * D + lane * PER, vw);
+          } else {
+            auto scatter = [&](T* dst, int64_t to) {
+#pragma unroll
+              for (int e = 0; e < PER; ++e) dst[vt_index(to, lane * PER + e, D)] = (uint16_t)(vw[e / 2] >> (16 * (e & 1)));
+            };
+            if (to_cache) scatter(reinterpret_cast<T*>(a.cache_vt) + bh * D * a.slot_stride, slot);
+            if (a.vt_out) scatter(reinterpret_cast<T*>(a.vt_out) + bh * D * a.chunk_stride, s);
+          }
+        }
       }
     }
   }
   if (!grouped) return;  // uniform over the workgroup
   __syncthreads();
-  // piece (head, d): the 8 tokens' values of dim d, 16 bytes at slot group slot_first / 8
-  for (int i = threadIdx.x; i < H * D; i += blockDim.x) {
+  // piece (head, d): the 8 tokens' values of dim d, 16 bytes at slot group first / 8
+  for (int i = threadIdx.x; i < H * D; i += kTileThreads) {
     const int hh = i / D, d = i - hh * D;
-    const u32x4 piece = reinterpret_cast<const u32x4*>(vt_lds)[i];
+    const uint16_t* col = v_lds + hh * kTileTok * D + d;
+    u32x4 piece;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) piece[j] = (uint32_t)col[2 * j * D] | ((uint32_t)col[(2 * j + 1) * D] << 16);
     const int64_t bh = (int64_t)b * H + hh;
-    if (tc_first)
-      *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(a.cache_vt) + bh * D * a.slot_stride + vt_index(slot_first, d, D)) = piece;
+    if (s0 >= drop)
+      *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(a.cache_vt) + bh * D * a.slot_stride + vt_index(first, d, D)) = piece;
     if (a.vt_out)
       *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(a.vt_out) + bh * D * a.chunk_stride + vt_index(s0, d, D)) = piece;
   }

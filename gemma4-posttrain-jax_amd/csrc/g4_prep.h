@@ -140,7 +140,14 @@ __device__ __forceinline__ void prep_math(PrepIn<BF16, D>& in, bool norm, bool h
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       const int d = lane * PER + e;
-      const float partner = __shfl_xor(in.x[e], PARTNER, 64);
+      float partner;
+      if constexpr (PARTNER == 32) {
+        const uint32_t u = __float_as_uint(in.x[e]);
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // the low / high half's value
+        partner = __uint_as_float(lane < 32 ? r[1] : r[0]);
+      } else {
+        partner = __shfl_xor(in.x[e], PARTNER, 64);
+      }
       const float rot = d < D / 2 ? -partner : partner;
       const float c = E::round(in.cv[e]);
       const float sn = E::round(in.sv[e]);
