@@ -139,7 +139,6 @@ PROTOTYPES = {
     "g4_softcap_bf16": (c_int32, [c_int64, c_void_p, c_float, c_void_p, c_void_p]),
     "g4_lm_head_sample_workspace_size": (c_size_t, [POINTER(G4LmHeadSampleArgs)]),
     "g4_lm_head_sample": (c_int32, [POINTER(G4LmHeadSampleArgs), c_void_p]),
-    "g4_lm_head_capped": (c_int32, [POINTER(G4LmHeadSampleArgs), c_void_p]),
     "g4_rms_norm": (c_int32, [c_int32, c_int32, c_int32, c_void_p, c_void_p, c_float, c_void_p, c_void_p]),
     "g4_residual_norm": (c_int32, [c_int32, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                    c_float, c_void_p, c_void_p, c_void_p]),

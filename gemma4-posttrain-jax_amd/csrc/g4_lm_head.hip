@@ -154,7 +154,7 @@ __device__ __forceinline__ void lh_compute(uint32_t slot, floatx4 (&acc)[4][LhSh
 // The epilogue of four consecutive columns n .. n + 3 of one row: bf16 rounding (the logits), the
 // optional logits store, the soft-cap, the running max / sum and the running argmax of the scores.
 // UNIT_T: temperature 1, no division (the compiler would otherwise divide every logit and select).
-template <bool SAMPLE, bool GREEDY, bool UNIT_T, bool CAP>
+template <bool SAMPLE, bool GREEDY, bool UNIT_T>
 __device__ __forceinline__ void lh_epilogue(floatx4 v, LhState& sr, int row, int n, const G4LmHeadSampleArgs& a,
                                             const CapTable& ct, uint32_t k0, uint32_t k1) {
   uint32_t bits[4];
@@ -162,7 +162,6 @@ __device__ __forceinline__ void lh_epilogue(floatx4 v, LhState& sr, int row, int
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     bits[j] = f32_to_bf16_bits(v[j]);
-    if constexpr (CAP) bits[j] = f32_to_bf16_bits(capped(bits[j], ct));
     x[j] = bf16_bits_to_f32(bits[j]);
   }
   if (a.logits_out) {
@@ -200,15 +199,13 @@ __device__ __forceinline__ void lh_epilogue(floatx4 v, LhState& sr, int row, int
 }
 
 // SAMPLE: run the sampler epilogue (else only the bf16 logits are written); GREEDY: no noise;
-// UNIT_T: temperature 1; CAP (without SAMPLE): the logits are stored soft-capped, through the samplers'
-// table of the formula, instead of read back and rewritten by a launch
-// of their own (62 us at 256 rows of V = 262144; the E2B-like step 4393 -> 4357 us).
-template <int ROWS, bool SAMPLE, bool GREEDY, bool UNIT_T = false, bool CAP = false>
+// UNIT_T: temperature 1.
+template <int ROWS, bool SAMPLE, bool GREEDY, bool UNIT_T = false>
 __global__ __launch_bounds__(kLhThreads, kLhWgPerCu) void lm_head_kernel(G4LmHeadSampleArgs a) {
   using S_ = LhShape<ROWS>;
   constexpr int kLhSlots = S_::SLOTS;
   __shared__ __attribute__((aligned(1024))) unsigned char ring[kLhSlots][S_::SLOT];
-  __shared__ uint16_t cap_tab[SAMPLE || CAP ? kCapTableEntries : 1];
+  __shared__ uint16_t cap_tab[SAMPLE ? kCapTableEntries : 1];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
@@ -235,7 +232,7 @@ __global__ __launch_bounds__(kLhThreads, kLhWgPerCu) void lm_head_kernel(G4LmHea
 #pragma unroll
   for (int rb = 0; rb < 4; ++rb) st[rb] = LhState{kF32Min, 0.f, -INFINITY, 0.f, 0x7fffffff};
   const CapTable ct = cap_table(cap_tab, a.softcap);
-  if ((SAMPLE || CAP) && a.softcap > 0.f) {  // the soft-cap table, complete before any DMA is issued
+  if (SAMPLE && a.softcap > 0.f) {  // the soft-cap table, complete before any DMA is issued
     cap_table_fill(cap_tab, a.softcap, threadIdx.x, kLhThreads);
     __syncthreads();
   }
@@ -283,7 +280,7 @@ __global__ __launch_bounds__(kLhThreads, kLhWgPerCu) void lm_head_kernel(G4LmHea
 #pragma unroll
           for (int i = 0; i + 1 < S_::CB; ++i) acc[rb][i] = acc[rb][i + 1];
           acc[rb][S_::CB - 1] = v;
-          lh_epilogue<SAMPLE, GREEDY, UNIT_T, CAP>(v, st[rb], row, n0 + 16 * (S_::CB * wc + cb) + 4 * grp, a, ct, k0, k1);
+          lh_epilogue<SAMPLE, GREEDY, UNIT_T>(v, st[rb], row, n0 + 16 * (S_::CB * wc + cb) + 4 * grp, a, ct, k0, k1);
         }
       }
     }
@@ -377,11 +374,9 @@ __global__ __launch_bounds__(kCombineThreads) void lm_head_combine_kernel(G4LmHe
 }
 
 template <int ROWS>
-void launch_lm_head(const G4LmHeadSampleArgs& a, bool cap, int grid, hipStream_t st) {
+void launch_lm_head(const G4LmHeadSampleArgs& a, int grid, hipStream_t st) {
   const dim3 g((unsigned)grid), b(kLhThreads);
-  if (cap)
-    hipLaunchKernelGGL((lm_head_kernel<ROWS, false, true, false, true>), g, b, 0, st, a);
-  else if (!a.token_out)
+  if (!a.token_out)
     hipLaunchKernelGGL((lm_head_kernel<ROWS, false, true>), g, b, 0, st, a);
   else if (!(a.temperature > 0.f))
     hipLaunchKernelGGL((lm_head_kernel<ROWS, true, true>), g, b, 0, st, a);
@@ -422,11 +417,8 @@ extern "C" size_t g4_lm_head_sample_workspace_size(const G4LmHeadSampleArgs* arg
   return (size_t)lh_grid(*args, dev) * kLhRows * 5u * 4u;
 }
 
-namespace g4 {
-namespace {
-
-// `cap`: the logits are stored after the soft-cap (no draw)
-int run_lm_head(const G4LmHeadSampleArgs* args, bool cap, void* stream) {
+extern "C" int g4_lm_head_sample(const G4LmHeadSampleArgs* args, void* stream) {
+  using namespace g4;
   if (!args) return fail(G4_ERR_INVALID, "g4_lm_head_sample: args is NULL");
   const G4LmHeadSampleArgs& a = *args;
   if (a.batch <= 0 || a.batch > kLhRows)
@@ -464,27 +456,13 @@ int run_lm_head(const G4LmHeadSampleArgs* args, bool cap, void* stream) {
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int rows = a.batch <= 64 ? 64 : a.batch <= 128 ? 128 : 256;
   if (rows == 64)
-    launch_lm_head<64>(a, cap, grid, st);
+    launch_lm_head<64>(a, grid, st);
   else if (rows == 128)
-    launch_lm_head<128>(a, cap, grid, st);
+    launch_lm_head<128>(a, grid, st);
   else
-    launch_lm_head<256>(a, cap, grid, st);
+    launch_lm_head<256>(a, grid, st);
   if (int rc = check_launch("g4_lm_head_sample")) return rc;
   if (!sample) return G4_OK;
   hipLaunchKernelGGL(lm_head_combine_kernel, dim3((unsigned)a.batch), dim3(kCombineThreads), 0, st, a, grid, rows);
   return check_launch("g4_lm_head_sample (combine)");
-}
-
-}  // namespace
-}  // namespace g4
-
-extern "C" int g4_lm_head_sample(const G4LmHeadSampleArgs* args, void* stream) {
-  return g4::run_lm_head(args, false, stream);
-}
-
-extern "C" int g4_lm_head_capped(const G4LmHeadSampleArgs* args, void* stream) {
-  using namespace g4;
-  if (args && (args->token_out || !(args->softcap > 0.f)))
-    return fail(G4_ERR_INVALID, "g4_lm_head_capped: needs softcap > 0 and no token_out");
-  return run_lm_head(args, true, stream);
 }

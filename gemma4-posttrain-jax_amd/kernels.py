@@ -529,8 +529,7 @@ def lm_head_supported(x: torch.Tensor, embed: torch.Tensor) -> bool:
 
 def _lm_head_call(x: torch.Tensor, embed: torch.Tensor, *, softcap: float | None, temperature: float,
                   key: torch.Tensor | None, split_key: bool, token_out: torch.Tensor | None,
-                  logp_out: torch.Tensor | None, logits_out: torch.Tensor | None,
-                  capped: bool = False) -> torch.Tensor | None:
+                  logp_out: torch.Tensor | None, logits_out: torch.Tensor | None) -> torch.Tensor | None:
     if not lm_head_supported(x, embed):
         raise ValueError(f"g4_lm_head_sample does not take x {tuple(x.shape)} {x.dtype} / embed "
                          f"{tuple(embed.shape)} {embed.dtype} (bf16, rows <= 256, vocab % 128, hidden % 32)")
@@ -554,22 +553,18 @@ def _lm_head_call(x: torch.Tensor, embed: torch.Tensor, *, softcap: float | None
     if need:
         ws = torch.empty(need // 4, dtype=torch.float32, device=dev)
         a.workspace, a.workspace_bytes = ws.data_ptr(), need
-    if capped:
-        _lib.check(_lib.lib().g4_lm_head_capped(ctypes.byref(a), _stream()), "g4_lm_head_capped")
-    else:
-        _lib.check(_lib.lib().g4_lm_head_sample(ctypes.byref(a), _stream()), "g4_lm_head_sample")
+    _lib.check(_lib.lib().g4_lm_head_sample(ctypes.byref(a), _stream()), "g4_lm_head_sample")
     return ws
 
 
-def lm_head(x: torch.Tensor, embed: torch.Tensor, *, out: torch.Tensor | None = None,
-            softcap: float | None = None) -> torch.Tensor:
+def lm_head(x: torch.Tensor, embed: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Tensor:
     """g4_lm_head_sample without sampling: ``bf16(x [B, M] . embed [V, M]^T)`` with f32 accumulation
-    (the logits before the soft-cap); with ``softcap`` g4_lm_head_capped, the logits after it."""
+    (the logits before the soft-cap)."""
 
     if out is None:
         out = torch.empty((x.shape[0], embed.shape[0]), dtype=torch.bfloat16, device=x.device)
-    _lm_head_call(x, embed, softcap=softcap, temperature=0.0, key=None, split_key=False, token_out=None,
-                  logp_out=None, logits_out=out, capped=softcap is not None)
+    _lm_head_call(x, embed, softcap=None, temperature=0.0, key=None, split_key=False, token_out=None,
+                  logp_out=None, logits_out=out)
     return out
 
 

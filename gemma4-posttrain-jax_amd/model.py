@@ -568,10 +568,10 @@ def forward_lm_head(embed_tokens: torch.Tensor, hidden: torch.Tensor, softcap: f
     x = hidden.reshape(B * S, M)
     if x.is_cuda and kernels.lm_head_supported(x, embed_tokens):
         # the decode batch (<= 256 rows): the native LM head, the GEMM g4_lm_head_sample runs when it
-        # samples in its epilogue, so a step's logits and its fused draw see the same bf16 values; the
-        # soft-cap is applied as they are stored
-        return kernels.lm_head(x.contiguous(), embed_tokens, softcap=softcap).reshape(B, S, -1)
-    logits = _proj(x, embed_tokens).reshape(B, S, -1)
+        # samples in its epilogue, so a step's logits and its fused draw see the same bf16 values
+        logits = kernels.lm_head(x.contiguous(), embed_tokens).reshape(B, S, -1)
+    else:
+        logits = _proj(x, embed_tokens).reshape(B, S, -1)
     if softcap is not None:
         if logits.dtype == torch.bfloat16 and logits.is_cuda and logits.is_contiguous():
             logits = kernels.softcap(logits, softcap, out=logits)  # one native pass, the same bits

@@ -360,10 +360,6 @@ typedef struct G4LmHeadSampleArgs {
 size_t g4_lm_head_sample_workspace_size(const G4LmHeadSampleArgs* args);
 int g4_lm_head_sample(const G4LmHeadSampleArgs* args, void* stream);
 
-/* The plain LM head (token_out NULL) with logits_out after the soft-cap: the same bits as
- * g4_lm_head_sample's logits put through g4_softcap_bf16. softcap > 0. */
-int g4_lm_head_capped(const G4LmHeadSampleArgs* args, void* stream);
-
 /*
  * Fused elementwise glue of the decoder layer (row-major [rows, cols] arrays, cols <= 4096 for
  * the norms; one pass each, the reference's rounding points kept). dtype = G4_DTYPE_*.

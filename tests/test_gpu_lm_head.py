@@ -64,19 +64,6 @@ def test_lm_head_logits(device, B, V, M):
     _check_logits(x, e, logits)
 
 
-# rows at the edges of the three workgroup shapes; logits far into the cap (scale 2) and NaN / inf among them
-@pytest.mark.parametrize("B,V,M,cap,scale", [(1, 128, 64, 30.0, 0.05), (64, 1024, 192, 30.0, 2.0), (65, 640, 64, 1.5, 2.0),
-                                             (128, 384, 96, 50.0, 0.05), (129, 2048, 256, 30.0, 2.0),
-                                             (256, 66048, 128, 30.0, 2.0)])
-def test_lm_head_capped_is_the_logits_then_softcap(device, B, V, M, cap, scale):
-    x, e = _operands(device, B, V, M, seed=B, scale=scale)
-    e[V // 2, 3] = float("nan")
-    e[V // 3, 1] = float("inf")
-    want = kernels.softcap(kernels.lm_head(x, e), cap)
-    got = kernels.lm_head(x, e, softcap=cap)
-    np.testing.assert_array_equal(got.view(torch.int16).cpu().numpy(), want.view(torch.int16).cpu().numpy())
-
-
 def _draw_and_check(device, B, V, M, temperature, cap, seed, key_words=(7, 123)):
     x, e = _operands(device, B, V, M, seed=seed)
     key = SMP.key_tensor(list(key_words), device)
