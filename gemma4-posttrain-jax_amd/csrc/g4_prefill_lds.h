@@ -459,42 +459,48 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
 
   // ---- rows with no valid key: the average of all S values ------------------------------------------
   // The reference's softmax over S equal fills is 1/S on every key, the same output for every such row
-  // of the pair. Wave w sums chunks w, w + NW, ... straight from memory (the same MFMA, the uniform
-  // probability in every column), the waves' sums meet in LDS, and each wave writes its masked rows:
+  // of the pair. Wave w forms dims 16 VT_W w .. of it straight from memory, chunk after chunk into one
+  // accumulator (the same MFMA, the uniform probability in every column: the bits that pass 2 over all S
+  // keys gives), kUniform loads at a time; the average meets in LDS and each wave writes its masked rows.
   // S D values read once per workgroup with a masked row, instead of both passes over all S keys (11
-  // prompts of 1999 left-padded tokens, window 512, with the pads' chunks skipped: 425 -> 177 us).
+  // prompts of 1999 left-padded tokens, window 512, with the pads' chunks skipped: 404 -> 186 us; a share
+  // of the keys per wave, added at the end, takes the same time but rounds differently).
   if (!any_masked) return;
-  float* usum = reinterpret_cast<float*>(&ring[0][0]);  // [NW][D], then the sum in row 0
+  float* usum = reinterpret_cast<float*>(&ring[0][0]);  // [D]
   const float p_uniform = round_bf16(1.0f / (float)S);
-  floatx4 uacc[S_::VT];
+  constexpr int kUniform = 16, UC = kUniform / S_::VT_W;  // loads in flight, the chunks they cover
+  const int u_last = (S - 1) >> 5;
+  floatx4 uacc[S_::VT_W];
 #pragma unroll
-  for (int i = 0; i < S_::VT; ++i) uacc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < S_::VT_W; ++i) uacc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-  for (int c = w; c <= (S - 1) >> 5; c += NW) {
-    float p[8];
+  for (int c = 0; c <= u_last; c += UC) {
+    u32x4 v[UC][S_::VT_W];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) p[e] = (c << 5) + 8 * grp + e < S ? p_uniform : 0.f;
-    const bf16x8 pu = as_bf16x8(u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
-                                      pack_bf16x2(p[6], p[7])});
-    u32x4 v[S_::VT];
+    for (int u = 0; u < UC; ++u)
+      if (c + u <= u_last) {
 #pragma unroll
-    for (int i = 0; i < S_::VT; ++i)
-      v[i] = buffer_load16(rv, v_lane, (uint32_t)c * (uint32_t)(64 * D) + 256u * i);
-    __builtin_amdgcn_sched_barrier(0);  // every load of the chunk requested before the first wait
+        for (int i = 0; i < S_::VT_W; ++i)
+          v[u][i] = buffer_load16(rv, v_lane, (uint32_t)(c + u) * (uint32_t)(64 * D) + 256u * (w * S_::VT_W + i));
+      }
+    __builtin_amdgcn_sched_barrier(0);  // every load of the group requested before the first wait
 #pragma unroll
-    for (int i = 0; i < S_::VT; ++i) uacc[i] = mfma16x16x32(as_bf16x8(v[i]), pu, uacc[i]);
+    for (int u = 0; u < UC; ++u)
+      if (c + u <= u_last) {
+        float p[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[e] = ((c + u) << 5) + 8 * grp + e < S ? p_uniform : 0.f;
+        const bf16x8 pu = as_bf16x8(u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
+                                          pack_bf16x2(p[6], p[7])});
+#pragma unroll
+        for (int i = 0; i < S_::VT_W; ++i) uacc[i] = mfma16x16x32(as_bf16x8(v[u][i]), pu, uacc[i]);
+      }
   }
   __syncthreads();  // every wave is done with the ring
   if (col == 0) {
 #pragma unroll
-    for (int i = 0; i < S_::VT; ++i) *reinterpret_cast<floatx4*>(usum + w * D + 16 * i + 4 * grp) = uacc[i];
-  }
-  __syncthreads();
-  for (int d = tid; d < D; d += NW * 64) {
-    float t = usum[d];
-#pragma unroll
-    for (int i = 1; i < NW; ++i) t += usum[i * D + d];
-    usum[d] = t;
+    for (int i = 0; i < S_::VT_W; ++i)
+      *reinterpret_cast<floatx4*>(usum + 16 * (w * S_::VT_W + i) + 4 * grp) = uacc[i];
   }
   __syncthreads();
 #pragma unroll

@@ -67,3 +67,20 @@ def test_prefill_group_sizes_padded(device, D, R):
     key_mask = np.ones((2, 100), bool)
     key_mask[1, :37] = False
     _check(device, 2, 100, 2, R, D, 0, key_mask, (0, 1), D + R)
+
+
+@pytest.mark.parametrize("D", [128, 256, 512])
+@pytest.mark.parametrize("S", [33, 161, 1999])
+def test_prefill_keyless_rows_sum_in_key_order(device, D, S):
+    """A row without a valid key averages all S values, summed in key order: bit for bit the last row of the
+    same values under scores that are all equal (q = 0: probabilities of 1 / S on every key)."""
+
+    g = torch.Generator(device="cuda").manual_seed(D + S)
+    H, R, Sp = 2, 4, (S + 63) // 64 * 64
+    k = torch.randn((1, H, Sp, D), device="cuda", generator=g).to(torch.bfloat16).expand(2, H, Sp, D)
+    v = torch.randn((1, H, Sp, D), device="cuda", generator=g).to(torch.bfloat16).expand(2, H, Sp, D)
+    q = torch.zeros((2, S, H, R, D), device="cuda", dtype=torch.bfloat16)
+    km = torch.tensor([[True], [False]], device=device).expand(2, S).contiguous()
+    out = kernels.prefill_attention(q, group_keys(k.contiguous()), group_values(v.contiguous()), km, window=0)
+    differ = int((out[1].view(torch.int16) != out[0, S - 1].view(torch.int16)).sum())
+    assert differ == 0
