@@ -212,7 +212,8 @@ def decode_attention(
         q_pos_scalar=qp_scalar, q_pos=qp_ptr, key_mask=_ptr(key_mask), key_mask_stride=key_mask.stride(0),
         q=_ptr(q), cache_k=_ptr(layer.key), cache_vt=_ptr(layer.value_t), cache_k_w=_ptr(layer.key),
         new_k=_ptr(new_k), new_v=_ptr(new_v), out=_ptr(out), workspace=None, workspace_bytes=0, prep=None,
-        num_splits=_decode_mode(num_splits, B * H, layer),
+        # no_alloc: the library's own choice, so that a call whose path needs no workspace shares no scratch
+        num_splits=num_splits if no_alloc else _decode_mode(num_splits, B * H, layer),
     )
     if no_alloc:
         _lib.check(_lib.lib().g4_decode_attention_noalloc(ctypes.byref(a), _stream()), "g4_decode_attention_noalloc")

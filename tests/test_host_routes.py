@@ -1,0 +1,61 @@
+"""Which native call the Python front end makes, and what it refuses, on the CPU: the launching entry points
+are replaced by recorders, the host-side ones are the library's."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from gemma4_posttrain_jax_amd import _lib, kernels
+from gemma4_posttrain_jax_amd.kvcache import new_layer_cache
+
+HOST_FUNCTIONS = ("g4_decode_workspace_size", "g4_linear_workspace_size", "g4_lm_head_sample_workspace_size")
+
+
+class _Recorder:
+    def __init__(self, native):
+        self.native, self.calls = native, []
+
+    def __getattr__(self, name):
+        if name in HOST_FUNCTIONS:
+            return getattr(self.native, name)
+
+        def launch(args, *rest):
+            copy = type(args._obj)()
+            ctypes.pointer(copy)[0] = args._obj
+            self.calls.append((name, copy))
+            return _lib.G4_OK
+
+        return launch
+
+
+@pytest.fixture
+def recorder(monkeypatch):
+    rec = _Recorder(_lib.lib())
+    monkeypatch.setattr(_lib, "lib", lambda: rec)
+    monkeypatch.setattr(kernels, "_ptr", lambda t: None if t is None else t.data_ptr())
+    monkeypatch.setattr(kernels, "_stream", lambda: None)
+    return rec
+
+
+def _decode(pairs, D=256, cap=512, **kw):
+    layer = new_layer_cache(pairs, 1, D, cap, True, torch.bfloat16, "cpu")
+    q = torch.zeros((pairs, 1, 4, D), dtype=torch.bfloat16)
+    mask = torch.ones((pairs, cap), dtype=torch.bool)
+    kernels.decode_attention(layer, q, mask, q_pos=cap - 1, window=cap, **kw)
+
+
+@pytest.mark.parametrize("pairs", [1, 2, 32, 129, 192, 255])
+def test_no_alloc_decode_shares_no_scratch_where_none_is_needed(recorder, pairs):
+    """Rows of at most 512 slots over fewer than 256 pairs have a path without a workspace: a no-alloc call
+    takes it (the library's per-device scratch would tie calls on different streams together); a call that
+    may allocate takes the two-launch path."""
+
+    _decode(pairs, no_alloc=True)
+    _decode(pairs)
+    (name, a), (_, b) = recorder.calls
+    assert name == "g4_decode_attention_noalloc"
+    assert a.num_splits == 0 and recorder.native.g4_decode_workspace_size(ctypes.byref(a)) == 0
+    assert b.num_splits == _lib.G4_DECODE_TWO_PASS and b.workspace and b.workspace_bytes > 0
