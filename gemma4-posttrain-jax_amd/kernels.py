@@ -254,6 +254,8 @@ def decode_attention_fused(
     if q_raw.dtype != layer.key.dtype or q_raw.stride(3) != 1 or (R > 1 and q_raw.stride(2) != D) or (
             H > 1 and q_raw.stride(1) != R * D):
         raise ValueError("q_raw must hold [Hkv, R, D] contiguous rows in the cache dtype")
+    if tuple(layer.key.shape[:2]) != (B, H) or layer.head_dim != D:
+        raise ValueError(f"cache {tuple(layer.key.shape)} does not match q_raw {tuple(q_raw.shape)}")
     for name, t in (("k_raw", k_raw), ("v_raw", v_raw)):
         if t is not None and (tuple(t.shape) != (B, H, D) or (B > 1 and t.stride(0) != stride)
                               or (H > 1 and t.stride(1) != D)

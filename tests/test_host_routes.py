@@ -59,3 +59,21 @@ def test_no_alloc_decode_shares_no_scratch_where_none_is_needed(recorder, pairs)
     assert name == "g4_decode_attention_noalloc"
     assert a.num_splits == 0 and recorder.native.g4_decode_workspace_size(ctypes.byref(a)) == 0
     assert b.num_splits == _lib.G4_DECODE_TWO_PASS and b.workspace and b.workspace_bytes > 0
+
+
+@pytest.mark.parametrize("cache", [dict(B=1), dict(H=1), dict(H=4), dict(D=128)])
+def test_fused_decode_refuses_a_cache_of_another_shape(recorder, cache):
+    """The step's fused attention refuses what its two calls, the append and the attention, refuse: a cache
+    whose rows, kv heads or head dim are not the query's (the kernels would index past it)."""
+
+    B, H, R, D = 2, 2, 4, 256
+    shape = dict(dict(B=B, H=H, D=D), **cache)
+    layer = new_layer_cache(shape["B"], shape["H"], shape["D"], 64, False, torch.bfloat16, "cpu")
+    rows = torch.zeros((B, (R + 2) * H * D), dtype=torch.bfloat16)
+    args = dict(q_pos=torch.zeros(B, dtype=torch.int32), window=0, k_raw=rows[:, R * H * D:-H * D].view(B, H, D),
+                v_raw=rows[:, -H * D:].view(B, H, D), q_norm_weight=None, k_norm_weight=None,
+                rope_cos=torch.zeros(B, D), rope_sin=torch.zeros(B, D), eps=1e-6, flags=0)
+    with pytest.raises(ValueError, match="does not match"):
+        kernels.decode_attention_fused(layer, rows[:, : R * H * D].view(B, H, R, D), torch.ones((B, 64), dtype=torch.bool),
+                                       **args)
+    assert not recorder.calls
