@@ -223,14 +223,16 @@ def _split_down(act: torch.Tensor, w_t: torch.Tensor) -> bool:
             and k % (64 * DOWN_KSPLIT) == 0 and act.is_contiguous() and w_t.is_contiguous())
 
 
-def _fused_decode_prep(x: torch.Tensor, pairs: int, head_dim: int, cache) -> bool:
+def _fused_decode_prep(x: torch.Tensor, pairs: int, head_dim: int, cache, norms=()) -> bool:
     """Whether a decode layer's q/k/v preparation and append run inside the two-launch attention
     (G4DecodePrep): rows of at most 1024 slots, head dims 128 / 256 / 512, bf16, at every number of
-    (b, kv head) pairs (one launch, the append's 4.6 us, fewer per layer; E2B step, with the two-launch
-    rows of 513 .. 1024 slots: 2.62 -> 2.46 ms at 1 row, 3.03 -> 2.9 ms at 64)."""
+    (b, kv head) ``pairs`` (one launch, the append's 4.6 us, fewer per layer; E2B step, with the two-launch
+    rows of 513 .. 1024 slots: 2.62 -> 2.46 ms at 1 row, 3.03 -> 2.9 ms at 64). It reads a lane's
+    ``head_dim / 64`` values of the q / k norm weights (``norms``) in one access; weights that start
+    elsewhere (a view into a larger buffer) take the append, which has a form for them."""
 
     return (x.dtype == torch.bfloat16 and head_dim in (128, 256, 512) and cache is not None
-            and cache.capacity <= 1024)
+            and cache.capacity <= 1024 and all(w is None or w.data_ptr() % (head_dim // 32) == 0 for w in norms))
 
 
 def _native_gate_up(h: torch.Tensor, w_t: torch.Tensor) -> bool:
@@ -452,7 +454,9 @@ def forward_gemma4_text(
         cos, sin = rot[lt]
         layer_cache = kv_cache.layers[i]
         shared = is_kv_shared(config, i)
-        if write_pos is not None and _fused_decode_prep(x, B * H, D, new_layers[sources[i]] if shared else layer_cache):
+        qk_norms = [n if n is None else n.weight for n in (lp.attention.q_norm, lp.attention.k_norm)]
+        if write_pos is not None and _fused_decode_prep(x, B * H, D, new_layers[sources[i]] if shared else layer_cache,
+                                                        qk_norms):
             # graphed decode step: g4_kv_append's work runs inside the
             # two-launch attention (G4DecodePrep) on the raw projection rows
             if shared:
@@ -465,8 +469,7 @@ def forward_gemma4_text(
                 new_layers.append(layer_cache)
             attn = kernels.decode_attention_fused(
                 src_cache, q[:, 0], key_mask, q_pos=slot, window=config.sliding_window, k_raw=kr, v_raw=vr,
-                q_norm_weight=lp.attention.q_norm.weight,
-                k_norm_weight=None if lp.attention.k_norm is None else lp.attention.k_norm.weight,
+                q_norm_weight=qk_norms[0], k_norm_weight=qk_norms[1],
                 rope_cos=cos[:, 0], rope_sin=sin[:, 0], eps=eps, flags=flags).view(B, 1, H, R, D)
         else:
             q_out = torch.empty((B, S, H, R, D), dtype=x.dtype, device=dev)

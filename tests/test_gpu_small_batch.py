@@ -8,9 +8,13 @@ import pytest
 import torch
 
 from gemma4_posttrain_jax_amd import _lib, kernels
+from gemma4_posttrain_jax_amd import config as C
+from gemma4_posttrain_jax_amd import model as M
+from gemma4_posttrain_jax_amd import sampler as SMP
 from gemma4_posttrain_jax_amd.kvcache import new_layer_cache
 from gemma4_posttrain_jax_amd.model import rotary_tables
 from oracle import g4_oracle as O
+from test_gpu_decode_prep import PREP_CFG
 from test_gpu_kernels import _decode_case
 
 pytestmark = pytest.mark.gpu
@@ -117,3 +121,28 @@ def test_lm_head_row_shapes(device, rows, vocab, hidden):
         want_tok, want_logp = kernels.sample_tokens(logits, **args)
         assert torch.equal(tok, want_tok)
         assert torch.all((logp - want_logp).abs() <= 2e-6)
+
+
+def test_step_with_norm_weights_at_odd_offsets(device, monkeypatch):
+    """A graphed step whose q / k norm weights are views at odd offsets of one buffer: the logits of the step
+    with weights of their own and the append run separately, bit for bit."""
+
+    cfg = C.config_from_hf(PREP_CFG)
+    params = M.params_from_numpy(O.init_params(O.config_from_hf(PREP_CFG), seed=5, dtype=O.BF16, std=0.03, norm_std=0.05,
+                                               layer_scalar_min=0.8), cfg, dtype=torch.bfloat16, device=device)
+
+    def moved(norm):
+        return norm and M.RMSNormParams(torch.cat([norm.weight[:1], norm.weight])[1:])
+
+    layers = [lp._replace(attention=lp.attention._replace(q_norm=moved(lp.attention.q_norm), k_norm=moved(lp.attention.k_norm)))
+              for lp in params.layers]
+    ids = torch.arange(24, dtype=torch.int32, device=device).view(2, 12) + 3
+    mask = torch.ones_like(ids, dtype=torch.bool)
+    active = torch.ones(2, dtype=torch.bool, device=device)
+    logits = []
+    for p in (params._replace(layers=tuple(layers)), params):
+        out = SMP.prefill(p, cfg, ids, mask, max_new_tokens=4)
+        engine = SMP.GraphedDecodeStep(p, cfg, out.kv_cache)
+        logits.append(engine.step(ids[:, 0], mask.sum(-1, dtype=torch.int32), active).clone())
+        monkeypatch.setattr(M, "_fused_decode_prep", lambda *args: False)
+    assert torch.equal(logits[0], logits[1])

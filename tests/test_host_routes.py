@@ -8,7 +8,7 @@ import ctypes
 import pytest
 import torch
 
-from gemma4_posttrain_jax_amd import _lib, kernels
+from gemma4_posttrain_jax_amd import _lib, kernels, model
 from gemma4_posttrain_jax_amd.kvcache import new_layer_cache
 
 HOST_FUNCTIONS = ("g4_decode_workspace_size", "g4_linear_workspace_size", "g4_lm_head_sample_workspace_size")
@@ -77,3 +77,25 @@ def test_fused_decode_refuses_a_cache_of_another_shape(recorder, cache):
         kernels.decode_attention_fused(layer, rows[:, : R * H * D].view(B, H, R, D), torch.ones((B, 64), dtype=torch.bool),
                                        **args)
     assert not recorder.calls
+
+
+@pytest.mark.parametrize("D", [128, 256, 512])
+def test_norm_weights_at_any_offset_take_the_append(recorder, D):
+    """The q / k norm weights may start anywhere (a view into a flat parameter buffer): the fused preparation
+    reads D / 64 of them in one access and refuses such a start, the append takes it."""
+
+    layer = new_layer_cache(1, 1, D, 64, False, torch.bfloat16, "cpu")
+    x, flat = torch.zeros((1, 1, 8), dtype=torch.bfloat16), torch.ones(D + 8, dtype=torch.bfloat16)
+    for offset, takes in ((0, True), (1, False), (D // 64, True)):
+        for norms in ((flat[offset:][:D], None), (flat[:D], flat[offset:][:D])):
+            assert model._fused_decode_prep(x, 1, D, layer, norms) is takes
+            prep = _lib.G4DecodePrep(q_raw=256, k_raw=256, v_raw=256, in_row_stride=3 * D, q_norm_weight=norms[0].data_ptr(),
+                                     k_norm_weight=norms[1].data_ptr() if norms[1] is not None else None, rope_cos=256,
+                                     rope_sin=256, eps=1e-6, flags=0)
+            a = _lib.G4DecodeArgs(dtype=_lib.G4_DTYPE_BF16, kind=_lib.G4_CACHE_LINEAR, batch=1, kv_heads=1, group=1,
+                                  head_dim=D, capacity=64, slot_stride=64, key_mask=256, key_mask_stride=64, cache_k=256,
+                                  cache_vt=256, cache_k_w=256, out=256, num_splits=0,
+                                  prep=ctypes.cast(ctypes.pointer(prep), ctypes.c_void_p))
+            # refused before any launch, or only for its missing workspace
+            want = _lib.G4_ERR_WORKSPACE if takes else _lib.G4_ERR_INVALID
+            assert recorder.native.g4_decode_attention(ctypes.byref(a), None) == want
