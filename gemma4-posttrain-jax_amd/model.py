@@ -260,14 +260,16 @@ def _mm(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
 
 def _native_proj(x: torch.Tensor, w_t: torch.Tensor) -> bool:
     """Whether a projection runs as g4_linear_bf16: a bf16 decode batch of at most 192 rows, and shapes its
-    few-row kernel streams in one round (every shape up to 64 rows). At 256 rows the library's tiles fill
+    few-row kernel streams in one round (every shape up to 64 rows), both operands as it loads them (16-byte
+    aligned; an embedding may be a view at any offset). At 256 rows the library's tiles fill
     (q/k/v 13.0 / 12.0 us, o 11.6 / 8.8) and it stays: 1 % of that step, for outputs that round from
     another f32 order."""
 
     (rows, k), n = x.shape, w_t.shape[0]
     return (x.is_cuda and x.dtype == torch.bfloat16 and w_t.dtype == torch.bfloat16 and 0 < rows <= 192
             and (rows <= 64 or (k <= 4096 and n < 4096)) and n % 64 == 0 and k % 64 == 0
-            and n * k < 2 ** 30 and x.is_contiguous() and w_t.is_contiguous())
+            and n * k < 2 ** 30 and rows * k < 2 ** 30 and x.is_contiguous() and w_t.is_contiguous()
+            and x.data_ptr() % 16 == 0 and w_t.data_ptr() % 16 == 0)
 
 
 def _proj(x: torch.Tensor, w_t: torch.Tensor) -> torch.Tensor:

@@ -146,3 +146,19 @@ def test_step_with_norm_weights_at_odd_offsets(device, monkeypatch):
         logits.append(engine.step(ids[:, 0], mask.sum(-1, dtype=torch.int32), active).clone())
         monkeypatch.setattr(M, "_fused_decode_prep", lambda *args: False)
     assert torch.equal(logits[0], logits[1])
+
+
+@pytest.mark.parametrize("moved", ["embed", "hidden"])
+def test_lm_head_fallback_takes_any_offset(device, moved):
+    """Logits of a vocabulary that the LM-head kernel does not take (no multiple of 128), from operands that
+    start at an odd element of a larger buffer: within the bf16 rounding of their f32 sums."""
+
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rows, vocab, hidden = 3, 192, 64
+    x = torch.randn((rows * hidden + 1,), device="cuda", generator=g).to(torch.bfloat16)[int(moved == "hidden"):]
+    e = torch.randn((vocab * hidden + 1,), device="cuda", generator=g).to(torch.bfloat16)[int(moved == "embed"):]
+    x, e = x[: rows * hidden].view(rows, 1, hidden), e[: vocab * hidden].view(vocab, hidden)
+    ref = x[:, 0].double() @ e.double().T
+    slack = 2.0 ** -20 * (x[:, 0].double().abs() @ e.double().abs().T)
+    got = M.forward_lm_head(e, x, None)[:, 0].double()
+    assert torch.all((got - ref).abs() <= ref.abs() * 2.0 ** -8 + slack)
