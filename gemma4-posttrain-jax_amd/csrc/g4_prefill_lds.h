@@ -6,16 +6,16 @@
 // V^T operand tile it reads from LDS feeds NB MFMAs. The key range is walked in 32-key chunks:
 // every chunk's K and V^T are DMA'd into LDS once per workgroup (buffer_load ... lds, each wave
 // issuing an equal share, into rings of 4 slots, 2 at head dim 512, where a chunk's operand is 32 KiB)
-// as lane-ordered MFMA operand tiles, and all waves read them from there (head dim 512, 4 x 1024 tokens:
-// 600 us with one wave per SIMD loading its own operands, 97 us here). The key-mask bytes of the row are staged in LDS once, so a chunk's validity
-// is one LDS byte per lane and a ballot.
+// as lane-ordered MFMA operand tiles, and all waves read them from there (head dim 512, 4 x 1024 tokens
+// without pads, 2 kv heads of 4: 630 us with one wave per SIMD loading its own operands, 102 us here). The
+// key-mask bytes of the row are staged in LDS once, so a chunk's validity is one LDS byte per lane and a ballot.
 //
 // Same two passes as prefill_bf16_kernel (the reference rounds probabilities after the full-row
 // softmax): pass 1 streams K for each row's max and sum, pass 2 streams K and V and forms the bf16
-// probabilities of the full-row softmax for the value product, evaluated as __expf(s - m) * (1/l):
-// the hardware exp and the row's reciprocal instead of expf and a division per score, a few f32
-// ulps from exp(s - m) / l, so a probability at a bf16 rounding boundary may round one bf16 step
-// the other way. Workgroups are launched heaviest (latest positions, longest causal key range)
+// probabilities of the full-row softmax for the value product, at head dims 128 and 256 evaluated as
+// __expf(s - m) * (1/l): the hardware exp and the row's reciprocal instead of expf and a division per score,
+// a few f32 ulps from exp(s - m) / l, so a probability at a bf16 rounding boundary may round one bf16 step
+// the other way (head dim 512: pf_exp, pf_prob). Workgroups are launched heaviest (latest positions, longest causal key range)
 // first.
 //
 // What bounds it is the issue rate of each SIMD's two waves, VALU work included, more than the
@@ -102,6 +102,36 @@ __device__ __forceinline__ void pf_pv(uint32_t vbase, const bf16x8 (&pop)[NB], f
     if (i + WIN < VT) vv[i % WIN] = lds_read16_at(vbase, 1024 * (i + WIN));
   }
   __builtin_amdgcn_sched_barrier(0);
+}
+
+// exp(x) for x <= 0 (NaN stays NaN) as 2^hi exp(r): hi = x log2(e) rounded, 2^hi from v_exp_f32, and
+// r = x - hi ln 2 by fmas with ln 2 in two parts, so that the rounding of hi does not enter (Cody and Waite's
+// reduction), exp(r) = 1 + r for |r| < 2^-17. About 1 ulp at any x, where __expf's error grows with |x|;
+// results below the smallest normal float are 0.
+__device__ __forceinline__ float exp_nonpos(float x) {
+  constexpr float kLog2e = 0x1.715476p+0f, kLn2Hi = 0x1.62e42ep-1f, kLn2Lo = 0x1.efa39ep-25f;
+  const float hi = x * kLog2e;
+  const float r = fmaf(-hi, kLn2Lo, fmaf(-hi, kLn2Hi, x));
+  const float e = __builtin_amdgcn_exp2f(hi);
+  return fmaf(e, fminf(r, 1.f), e);  // (x at the lowest bf16, a masked key: hi = -inf, r = inf, e = 0)
+}
+
+// The softmax's exp and a probability exp(x) / sum. Head dims 128 and 256: the hardware exp and the row's
+// reciprocal (see the head of this file). Head dim 512 keeps the precision of prefill_bf16_kernel's expf and
+// division, which its rows took before (4 x 1024 tokens: 100.1 us with the other head dims' two, 102.3 with
+// these, about 118 with expf and a division).
+template <int D>
+__device__ __forceinline__ float pf_exp(float x) {
+  if constexpr (D == 512) return exp_nonpos(x);
+  return __expf(x);
+}
+template <int D>
+__device__ __forceinline__ float pf_prob(float x, float sum, float rsum) {
+  if constexpr (D == 512) {  // the quotient from the reciprocal with one residual correction (Markstein)
+    const float e = exp_nonpos(x), q = e * rsum;
+    return fmaf(fmaf(-q, sum, e), rsum, q);
+  }
+  return __expf(x) * rsum;
 }
 
 template <int D, int NB, int NW>
@@ -289,8 +319,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
         const float mn = fmaxf(m[cb], mx);
         float sum = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sum += __expf(sc[e] - mn);
-        l[cb] = l[cb] * __expf(m[cb] - mn) + sum;
+        for (int e = 0; e < 8; ++e) sum += pf_exp<D>(sc[e] - mn);
+        l[cb] = l[cb] * pf_exp<D>(m[cb] - mn) + sum;
         m[cb] = mn;
       }
       return;
@@ -307,8 +337,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
       const float mn = fmaxf(m[cb], mx);
       float sum = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sum += __expf(sc[e] - mn);
-      l[cb] = l[cb] * __expf(m[cb] - mn) + sum;
+      for (int e = 0; e < 8; ++e) sum += pf_exp<D>(sc[e] - mn);
+      l[cb] = l[cb] * pf_exp<D>(m[cb] - mn) + sum;
       m[cb] = mn;
     }
   };
@@ -342,7 +372,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
       const float m2 = __shfl_xor(m[cb], msk, 64);
       const float l2 = __shfl_xor(l[cb], msk, 64);
       const float mm = fmaxf(m[cb], m2);
-      l[cb] = l[cb] * __expf(m[cb] - mm) + l2 * __expf(m2 - mm);
+      l[cb] = l[cb] * pf_exp<D>(m[cb] - mm) + l2 * pf_exp<D>(m2 - mm);
       m[cb] = mm;
     }
     // A row with no valid key is the reference's softmax over S equal fills: 1/S on every key.
@@ -370,8 +400,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t sw = pack_bf16x2(acc[cb][j >> 1][2 * (j & 1)], acc[cb][j >> 1][2 * (j & 1) + 1]);
-          pw[j] = pack_bf16x2(__expf(__uint_as_float(sw << 16) - m[cb]) * rl[cb],
-                              __expf(__uint_as_float(sw & 0xffff0000u) - m[cb]) * rl[cb]);
+          pw[j] = pack_bf16x2(pf_prob<D>(__uint_as_float(sw << 16) - m[cb], l[cb], rl[cb]),
+                              pf_prob<D>(__uint_as_float(sw & 0xffff0000u) - m[cb], l[cb], rl[cb]));
         }
         // (keeps the packing here: sunk below the branches, eight floats per block stay live over them)
         __asm__ volatile("" : "+v"(pw[0]), "+v"(pw[1]), "+v"(pw[2]), "+v"(pw[3]));
@@ -380,8 +410,8 @@ __global__ __launch_bounds__(NW * 64) void prefill_bf16_lds_kernel(G4PrefillArgs
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t sw = pack_bf16x2(acc[cb][j >> 1][2 * (j & 1)], acc[cb][j >> 1][2 * (j & 1) + 1]);
-          const float p0 = __expf(__uint_as_float(sw << 16) - m[cb]) * rl[cb];
-          const float p1 = __expf(__uint_as_float(sw & 0xffff0000u) - m[cb]) * rl[cb];
+          const float p0 = pf_prob<D>(__uint_as_float(sw << 16) - m[cb], l[cb], rl[cb]);
+          const float p1 = pf_prob<D>(__uint_as_float(sw & 0xffff0000u) - m[cb], l[cb], rl[cb]);
           pw[j] = pack_bf16x2((bits >> (2 * j)) & 1u ? p0 : 0.f, (bits >> (2 * j + 1)) & 1u ? p1 : 0.f);
         }
       }

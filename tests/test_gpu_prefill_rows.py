@@ -84,3 +84,31 @@ def test_prefill_keyless_rows_sum_in_key_order(device, D, S):
     out = kernels.prefill_attention(q, group_keys(k.contiguous()), group_values(v.contiguous()), km, window=0)
     differ = int((out[1].view(torch.int16) != out[0, S - 1].view(torch.int16)).sum())
     assert differ == 0
+
+
+def test_prefill_head_dim_512_probabilities(device):
+    """The bf16 probabilities themselves: scores that are exact in bf16 (one nonzero dim, q = 1), a few near 0
+    that make every row's sum another and the others 45 .. 80 below, and one-hot values, so that output dim j
+    is key j's probability.
+    Against the 64-bit softmax rounded once: an f32 exp, sum and division within 2.5 ulp (3e-7) cross a bf16
+    rounding boundary (at least 2^-8 of the value apart) for a share of at most 3e-7 * 2^8 = 7.7e-5 of them;
+    the rounding of x log2(e) alone (up to 2.6e-6 there, half of it on average) gives three times that."""
+
+    B, H, D = 64, 8, 512
+    S = D
+    g = torch.Generator(device="cuda").manual_seed(3)
+    k0 = (torch.rand((B, H, S), device="cuda", generator=g) * -35 - 45).to(torch.bfloat16)
+    k0[..., 0] = 0
+    k0[..., 1:9] = -2 * torch.rand((B, H, 8), device="cuda", generator=g).to(torch.bfloat16)
+    k = torch.zeros((B, H, S, D), device="cuda", dtype=torch.bfloat16)
+    k[..., 0] = k0
+    q = torch.zeros((B, S, H, 1, D), device="cuda", dtype=torch.bfloat16)
+    q[..., 0] = 1
+    v = torch.eye(S, device="cuda", dtype=torch.bfloat16).expand(B, H, S, D).contiguous()
+    km = torch.ones((B, S), dtype=torch.bool, device=device)
+    got = kernels.prefill_attention(q, group_keys(k), group_values(v), km, window=0)[:, -1, :, 0]  # [B, H, key]
+    want = torch.softmax(k0.double(), -1).to(torch.bfloat16)
+    share = float((got != want).float().mean())
+    print(f"share of probabilities that round the other way: {share:.2e}")
+    assert torch.all((got.double() - want.double()).abs() <= want.double() * 2.0 ** -7)
+    assert share <= 7.7e-5
