@@ -209,11 +209,8 @@ constexpr int kLdsBytes = 160 * 1024;  // gfx950 LDS per workgroup
 // one wave per SIMD with three or four blocks, which reuse each LDS tile more but leave a lone wave to
 // overlap its own MFMA, LDS and vector work: 1.85 ms vs 2.04 / 2.66 ms for 8 x 4096 tokens). Head dim
 // 512 holds twice the q and output registers per column block: four waves of two blocks, one wave per
-// SIMD. At head dim 128 one block per wave takes 94 registers and 66 KiB of LDS, so two workgroups share
-// a CU and each fills the other's barriers (8 x 4096 tokens, causal 507 -> 479 us, window 512 178 ->
-// 148; 8 x 2000 192 -> 137).
-template <int D>
-constexpr int pf_blocks() { return D == 128 ? 1 : 2; }  // 16-row column blocks per wave
+// SIMD.
+constexpr int kPfBlocks = 2;  // 16-row column blocks per wave, or one (pf_one_block)
 template <int D>
 constexpr int pf_waves() { return D == 512 ? 4 : 8; }  // waves per workgroup
 
@@ -224,6 +221,27 @@ constexpr int pf_waves() { return D == 512 ? 4 : 8; }  // waves per workgroup
 // and one round lasts as long as its last block, while two rounds pair long blocks with short ones
 // (1 x 1024: 88.9 -> 61.3 us; 4 x 1024 at head dim 512: 117.5 -> 84.9).
 constexpr int kPfFewGroups = 256;
+
+// Head dim 128, rows of up to kPfPairSeq keys: one block per wave takes 93 registers and 64 KiB + a byte per
+// key of LDS, so two workgroups share a CU and each fills the other's barriers (us, two blocks -> one: 8 x 4096
+// tokens of 2 x 4 heads, causal 505 -> 491, window 512 181 -> 156; 7 x 1100 of 4 x 8, causal 169 -> 153; 5 x
+// 3000 of 2 x 4, causal 221 -> 199). Not where two-block workgroups just fill two rounds of the CUs with long
+// causal rows (481 .. 512 of them: 1 x 8192 of 4 x 4 heads 506 / 537, 2 x 16000 of 1 x 4 939 / 1016; at 470
+// or 750 of them, or 1024 tokens, one block is as fast or faster). Beyond kPfPairSeq one workgroup has the CU,
+// and two blocks reuse each LDS tile twice (1 x 32768 of 1 x 4 heads, causal 2606 -> 1983, window 512 174 ->
+// 123; 1 x 18000 of 8 x 4, window 1024 879 -> 721), but for few groups: causal up to 5/4 of the CUs (282: 1373
+// / 940; 313: 1376 / 1109; 375: 1342 / 1548 with one), windowed up to half of them as above.
+constexpr int kPfPairSeq = 16000;
+
+// Whether a grid of `groups` two-block workgroups runs as one-block ones.
+template <int D>
+bool pf_one_block(const G4PrefillArgs& a, int64_t groups) {
+  const bool causal = a.window <= 0 || a.window >= a.seq;
+  if (D == 128 && a.seq <= kPfPairSeq)
+    return !(causal && a.seq > 1024 && groups > 2 * kPfFewGroups * 15 / 16 && groups <= 2 * kPfFewGroups);
+  if (!causal) return groups <= kPfFewGroups / 2;
+  return groups <= (D == 128 ? kPfFewGroups * 5 / 4 : kPfFewGroups);
+}
 
 // Largest key-mask row (bytes) the LDS-staged kernel of head dim 128 / 256 / 512 can hold next to its
 // static tile buffers on each device; 0 when the limit could not be raised. Written once per device
@@ -238,7 +256,7 @@ int raise_prefill_lds_limit(int device) {
   int& max_seq = g_lds_max_seq[device][pf_index<D>()];
   max_seq = kPfMaxSeq;
   const void* kernels[] = {(const void*)prefill_bf16_lds_kernel<D, 1, pf_waves<D>()>,
-                           (const void*)prefill_bf16_lds_kernel<D, pf_blocks<D>(), pf_waves<D>()>};
+                           (const void*)prefill_bf16_lds_kernel<D, kPfBlocks, pf_waves<D>()>};
   for (const void* fn : kernels) {
     hipFuncAttributes attr;
     int cap = 0;
@@ -263,16 +281,14 @@ void launch_prefill_blocks(const G4PrefillArgs& a, int64_t groups, hipStream_t s
 
 template <int D>
 void launch_prefill_lds(const G4PrefillArgs& a, hipStream_t st) {
-  constexpr int NB = pf_blocks<D>();
   const auto groups = [&](int nb) -> int64_t {  // workgroups of nb column blocks per wave
     const int ppb = pf_waves<D>() * nb * (16 / a.group);
     return (int64_t)((a.seq + ppb - 1) / ppb) * a.kv_heads * a.batch;
   };
-  const bool causal = a.window <= 0 || a.window >= a.seq;
-  if (NB == 1 || groups(NB) <= (causal ? kPfFewGroups : kPfFewGroups / 2))
+  if (pf_one_block<D>(a, groups(kPfBlocks)))
     launch_prefill_blocks<D, 1>(a, groups(1), st);
   else
-    launch_prefill_blocks<D, NB>(a, groups(NB), st);
+    launch_prefill_blocks<D, kPfBlocks>(a, groups(kPfBlocks), st);
 }
 
 }  // namespace

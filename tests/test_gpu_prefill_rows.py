@@ -112,3 +112,31 @@ def test_prefill_head_dim_512_probabilities(device):
     print(f"share of probabilities that round the other way: {share:.2e}")
     assert torch.all((got.double() - want.double()).abs() <= want.double() * 2.0 ** -7)
     assert share <= 7.7e-5
+
+
+# a grid whose workgroups hold two column blocks per wave, its heads one by one with one block: head dim 128 at
+# 512 two-block workgroups of more than 1024 tokens, beyond 16000 keys, and head dim 256 beyond 256
+@pytest.mark.parametrize("D,B,S,H,R,window", [(128, 4, 2048, 4, 4, 0), (128, 1, 16001, 8, 1, 0), (128, 1, 16001, 8, 1, 600),
+                                              (256, 5, 1025, 4, 4, 0)])
+def test_prefill_block_counts_agree(device, D, B, S, H, R, window):
+    """Rows do not depend on how many column blocks a workgroup holds: bit for bit the same; and the last
+    position within 2e-2 of 64 bits (the rounding of probabilities and outputs, |o| < 4)."""
+
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    Sp = (S + 63) // 64 * 64
+    q = (torch.randn((B, S, H, R, D), device="cuda", generator=g) * D ** -0.25).to(torch.bfloat16)
+    k = (torch.randn((B, H, Sp, D), device="cuda", generator=g) * D ** -0.25).to(torch.bfloat16)
+    v = torch.randn((B, H, Sp, D), device="cuda", generator=g).to(torch.bfloat16)
+    km = torch.ones((B, S), dtype=torch.bool, device=device)
+    km[0, :40] = False
+    kk, vv = group_keys(k), group_values(v)
+    out = kernels.prefill_attention(q, kk, vv, km, window=window)
+    for b in range(B):
+        for h in range(H):
+            one = kernels.prefill_attention(q[b:b + 1, :, h:h + 1].contiguous(), kk[b:b + 1, h:h + 1].contiguous(),
+                                            vv[b:b + 1, h:h + 1].contiguous(), km[b:b + 1], window=window)
+            assert int((one.view(torch.int16) != out[b:b + 1, :, h:h + 1].view(torch.int16)).sum()) == 0
+    seen = km & (torch.arange(S, device=device) > S - 1 - window if window else True)
+    scores = torch.matmul(q[:, -1].double(), k[:, :, :S].double().transpose(2, 3).contiguous())
+    want = torch.matmul(torch.softmax(scores.masked_fill(~seen[:, None, None], float("-inf")), -1), v[:, :, :S].double())
+    assert float((out[:, -1].double() - want).abs().max()) <= 2e-2
