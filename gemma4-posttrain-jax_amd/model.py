@@ -258,17 +258,35 @@ def _mm(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     return a @ b
 
 
+def _native_proj_k(rows: int, n: int) -> int:
+    """The longest K up to which the few-row GEMM is the faster one for ``rows`` (at most 192) x ``n`` outputs (0:
+    none). Library / native, us, weights from memory, N 256 .. 16384 by K 640 .. 8192 at 1 .. 192 rows:
+    - from 4096 columns one wave walks all of K: N = 4096 at 1 / 64 rows 15.4 / 18.6, 24.2 / 33.0 at K = 8192,
+      14.9 / 17.9 at 64 rows and K = 4096; N = 10240 leaves a last round a quarter full, 21.4 / 22.8 at 32 rows
+      and K = 4096;
+    - below, four waves share it: N = 2048 at 40 rows 13.8 / 14.7 at K = 8192;
+    - from 65 rows tiles that the columns do not fill: N = 1152 at 128 rows 10.2 / 11.9 at K = 3072, N = 2816 at
+      144 rows 11.9 / 13.6 at K = 2048."""
+
+    if n >= 4096:
+        return 2048 if rows > (16 if 8192 < n < 16384 else 32) else 5376 if rows <= 24 else 4096
+    if rows <= 64:
+        return 16384 if rows <= 16 else 8192 if rows <= 32 else 5376
+    if rows > 128 and n > 2560 and n % 512:
+        return 0
+    return 4096 if n % 256 == 0 or (n < 1152 and rows <= 128) else 2048
+
+
 def _native_proj(x: torch.Tensor, w_t: torch.Tensor) -> bool:
-    """Whether a projection runs as g4_linear_bf16: a bf16 decode batch of at most 192 rows, and shapes its
-    few-row kernel streams in one round (every shape up to 64 rows), both operands as it loads them (16-byte
-    aligned; an embedding may be a view at any offset). At 256 rows the library's tiles fill
-    (q/k/v 13.0 / 12.0 us, o 11.6 / 8.8) and it stays: 1 % of that step, for outputs that round from
-    another f32 order."""
+    """Whether a projection runs as g4_linear_bf16: a bf16 decode batch of at most 192 rows (64 from 4096
+    columns), shapes where its few-row kernel is the faster one, and both operands as it loads them (16-byte
+    aligned; an embedding may be a view at any offset). At 256 rows the library's tiles fill (q/k/v 13.0 / 12.0
+    us, o 11.6 / 8.8) and it stays: 132 us, 3 % of that step, for outputs that round from another f32 order."""
 
     (rows, k), n = x.shape, w_t.shape[0]
-    return (x.is_cuda and x.dtype == torch.bfloat16 and w_t.dtype == torch.bfloat16 and 0 < rows <= 192
-            and (rows <= 64 or (k <= 4096 and n < 4096)) and n % 64 == 0 and k % 64 == 0
-            and n * k < 2 ** 30 and rows * k < 2 ** 30 and x.is_contiguous() and w_t.is_contiguous()
+    return (x.is_cuda and x.dtype == torch.bfloat16 and w_t.dtype == torch.bfloat16
+            and 0 < rows <= (64 if n >= 4096 else 192) and k <= _native_proj_k(rows, n) and n % 64 == 0 and k % 64 == 0
+            and n * k < 2 ** 30 and x.is_contiguous() and w_t.is_contiguous()
             and x.data_ptr() % 16 == 0 and w_t.data_ptr() % 16 == 0)
 
 

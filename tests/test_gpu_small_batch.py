@@ -162,3 +162,24 @@ def test_lm_head_fallback_takes_any_offset(device, moved):
     slack = 2.0 ** -20 * (x[:, 0].double().abs() @ e.double().abs().T)
     got = M.forward_lm_head(e, x, None)[:, 0].double()
     assert torch.all((got - ref).abs() <= ref.abs() * 2.0 ** -8 + slack)
+
+
+# both sides of each line of _native_proj_k: (rows, N, K) that it takes, and the first beyond
+@pytest.mark.parametrize("rows,n,k,native", [
+    (24, 4096, 5376, True), (25, 4096, 5376, False), (32, 4096, 4096, True), (33, 4096, 4096, False),
+    (64, 4096, 2048, True), (65, 4096, 2048, False), (16, 8256, 2112, True), (17, 8256, 2112, False),
+    (16, 192, 16384, True), (17, 192, 16384, False), (32, 192, 8192, True), (33, 192, 8192, False),
+    (64, 192, 5376, True), (65, 192, 5376, False), (128, 1088, 4096, True), (129, 1088, 4096, False),
+    (192, 1152, 2048, True), (192, 1152, 2112, False), (192, 2560, 4096, True), (193, 2560, 4096, False),
+    (128, 2816, 640, True), (129, 2816, 640, False), (192, 3072, 640, True)])
+def test_projection_routes(device, rows, n, k, native):
+    """A projection takes the few-row GEMM where that was measured faster, the library's product beyond;
+    either within the bf16 rounding of its f32 sums."""
+
+    g = torch.Generator(device="cuda").manual_seed(rows + n)
+    x = torch.randn((rows, k), device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn((n, k), device="cuda", generator=g) * k ** -0.5).to(torch.bfloat16)
+    assert M._native_proj(x, w) is native
+    ref = x.double() @ w.double().T
+    slack = 2.0 ** -20 * (x.double().abs() @ w.double().abs().T)  # f32 sums of k products in any order
+    assert torch.all((M._proj(x, w).double() - ref).abs() <= ref.abs() * 2.0 ** -8 + slack)
