@@ -471,6 +471,15 @@ void launch_skinny_wide(const G4LinearArgs& a, float* partials, hipStream_t st) 
     launch_skinny<1, CB, 8>(a, partials, st);
 }
 
+// Rows up to which it takes a shape of many columns. Its workgroups (32 columns, 40 KiB of LDS) sit four to a
+// CU; where their last round is less than half full and long, the ring kernel is as fast from 57 rows (us at 48
+// / 64 rows, ring kernel / this: 43008 x 5376 134.5 / 128.7, 138.5 / 142.4; x 4096 108 / 100, 109 / 107;
+// at 49152 x 4096 116 / 113, 32768 x 5376 96 / 80 at 64 rows).
+int skinny_wide_rows(const G4LinearArgs& a) {
+  const int groups = a.n / 32;
+  return a.k > 4096 && groups >= 1152 && groups < 1536 ? 56 : kSkinnyRows;
+}
+
 // The tile (16 CB columns x 8 XG rows) whose workgroups bring the least through each of the 256 CUs:
 // cost = ceil(workgroups / 256) x (2 CB + XG) KiB per line.
 struct SkinnyTile {
@@ -558,7 +567,7 @@ extern "C" int g4_linear_bf16(const G4LinearArgs* args, void* stream) {
   // the gated GELU's products are the plain call's bit for bit); else 128 x 128 tiles when the rows fill
   // two halves and the columns divide by 128; else 256 x 64
   const bool wide = a.n >= kSkinnyWideCols && a.ksplit == 1;
-  if (wide && a.m <= kSkinnyRows) {
+  if (wide && a.m <= skinny_wide_rows(a)) {
     if (a.n / 16 <= 512)
       launch_skinny_wide<1>(a, partials, st);
     else

@@ -99,6 +99,21 @@ def test_few_row_linear(device, rows, n, k):
     assert torch.all((got - want).abs() <= bar)
 
 
+@pytest.mark.parametrize("n,k,rows", [(4096, 192, 64), (36864, 4160, 56)])
+def test_many_columns_keep_the_order_of_their_sums(device, n, k, rows):
+    """Many columns: the streaming kernel's last batch and the ring kernel's first give a row the same bits."""
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn((rows + 1, k), device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn((n, k), device="cuda", generator=g) * k ** -0.5).to(torch.bfloat16)
+    for call in (kernels.linear, kernels.linear_gelu):
+        few, more = call(x[:rows], w), call(x, w)
+        assert int((few.view(torch.int16) != more[:rows].view(torch.int16)).sum()) == 0
+    ref = x.double() @ w.double().T
+    slack = 2.0 ** -20 * (x.double().abs() @ w.double().abs().T)
+    assert torch.all((kernels.linear(x, w).double() - ref).abs() <= ref.abs() * 2.0 ** -8 + slack)
+
+
 # the last batch of each row shape (64, 128, 256 rows per workgroup) and the first of the next
 @pytest.mark.parametrize("rows", [1, 63, 64, 65, 128, 129])
 @pytest.mark.parametrize("vocab,hidden", [(128, 32), (1280, 96)])
