@@ -198,3 +198,27 @@ def test_projection_routes(device, rows, n, k, native):
     ref = x.double() @ w.double().T
     slack = 2.0 ** -20 * (x.double().abs() @ w.double().abs().T)  # f32 sums of k products in any order
     assert torch.all((M._proj(x, w).double() - ref).abs() <= ref.abs() * 2.0 ** -8 + slack)
+
+
+def test_lm_head_fallback_keeps_its_derivatives(device):
+    """Logits of a vocabulary that the LM-head kernel does not take (no multiple of 128) are the library's
+    product wherever a derivative or a transform follows them: reverse and forward mode, vmap."""
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.randn((4, 1, 64), device="cuda", generator=g).to(torch.bfloat16)
+    e = torch.randn((192, 64), device="cuda", generator=g).to(torch.bfloat16)
+    want = M.forward_lm_head(e, x, None)
+    with torch.no_grad():
+        assert M._native_proj(x[:, 0].contiguous(), e)
+    for operand in (x, e):
+        leaf = operand.clone().requires_grad_()
+        logits = M.forward_lm_head(leaf if operand is e else e, leaf if operand is x else x, None)
+        (grad,) = torch.autograd.grad(logits.float().sum(), leaf)
+        ref = e.float().sum(0).expand(4, 1, 64) if operand is x else x.float().sum((0, 1)).expand(192, 64)
+        assert torch.allclose(grad.float(), ref, rtol=2.0 ** -7, atol=2.0 ** -4)
+    tangent = torch.ones_like(x)
+    value, jvp = torch.func.jvp(lambda h: M.forward_lm_head(e, h, None), (x,), (tangent,))
+    assert torch.allclose(jvp.float(), M.forward_lm_head(e, tangent, None).float(), rtol=2.0 ** -7, atol=2.0 ** -4)
+    assert torch.allclose(value.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -4)
+    stacked = torch.func.vmap(lambda h: M.forward_lm_head(e, h[None], None)[0])(x)
+    assert torch.allclose(stacked.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -4)
