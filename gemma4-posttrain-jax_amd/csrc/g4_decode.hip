@@ -266,8 +266,10 @@ int launch_split_keys(const G4DecodeArgs& a, hipStream_t st) {
 // Where the automatic choice takes the two-launch path (us per call, D = 256, R = 4, HIP graph over 12
 // caches):
 // - rows of 513 .. 1024 slots: always (768 slots, three split-K launches before: 2 pairs 18.3 -> 10.7,
-//   64 pairs 22.5 -> 15.9, 128 pairs 30.6 -> 24.2, 192 pairs 42.6 -> 32.7), and every row at head dim
-//   512, which has no one-launch kernel;
+//   64 pairs 22.5 -> 15.9, 128 pairs 30.6 -> 24.2, 192 pairs 42.6 -> 32.7; at 1 / 64 / 255 pairs D = 128
+//   14.2 -> 9.6, 17.8 -> 12.8, 31.4 -> 24.6, D = 256, R = 16 25.1 -> 16.3, 33.6 -> 21.1, 85.3 -> 56.6; the
+//   narrowest gains are those of 1024 slots at R = 1 and 224 pairs, D = 128 30.5 -> 28.9, D = 256 49.0 -> 48.1),
+//   and every row at head dim 512, which has no one-launch kernel;
 // - rows of at most 512 slots from 256 pairs (one launch 71.8, two 62.9 at 512 pairs). With fewer, one
 //   launch needs no workspace, and the automatic choice keeps to it; callers that hold a workspace
 //   can ask for two launches where those are faster (kernels.decode_attention does).

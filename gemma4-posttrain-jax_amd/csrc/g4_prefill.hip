@@ -215,11 +215,12 @@ template <int D>
 constexpr int pf_waves() { return D == 512 ? 4 : 8; }  // waves per workgroup
 
 // Where two-block workgroups would leave CUs idle, one-block ones run instead, twice as many with
-// half the positions each and a shorter chunk step (2.55 -> 1.77 us per chunk at head dim 256, 3.6 ->
-// 2.4 at 512). Windowed rows: up to half the 256 CUs' count (1 x 4096 tokens, 2 kv heads, window 512:
-// 62.9 -> 45.5 us). Causal rows: up to the CU count, since the cost of a block grows with its position
+// half the positions each and a shorter chunk step (both passes: 2.9 -> 2.1 us per chunk at head dim 256,
+// 4.0 -> 2.7 at 512). Windowed rows: up to half the 256 CUs' count (1 x 4096 tokens of 2 x 4 heads, window
+// 512: 67.3 -> 50.4 us). Causal rows: up to the CU count, since the cost of a block grows with its position
 // and one round lasts as long as its last block, while two rounds pair long blocks with short ones
-// (1 x 1024: 88.9 -> 61.3 us; 4 x 1024 at head dim 512: 117.5 -> 84.9).
+// (2 x 4 heads, no pads: 1 x 1024 94.0 -> 67.2 us, 8 x 1024 96.7 -> 81.2; at head dim 512 1 x 1024 126.8 ->
+// 86.6, 4 x 1024 135.7 -> 106.5).
 constexpr int kPfFewGroups = 256;
 
 // Head dim 128, rows of up to kPfPairSeq keys: one block per wave takes 93 registers and 64 KiB + a byte per

@@ -7,7 +7,7 @@
 // every chunk's K and V^T are DMA'd into LDS once per workgroup (buffer_load ... lds, each wave
 // issuing an equal share, into rings of 4 slots, 2 at head dim 512, where a chunk's operand is 32 KiB)
 // as lane-ordered MFMA operand tiles, and all waves read them from there (head dim 512, 4 x 1024 tokens
-// without pads, 2 kv heads of 4: 630 us with one wave per SIMD loading its own operands, 102 us here). The
+// without pads, 2 kv heads of 4: 630 us with one wave per SIMD loading its own operands, 102-106 us here). The
 // key-mask bytes of the row are staged in LDS once, so a chunk's validity is one LDS byte per lane and a ballot.
 //
 // Same two passes as prefill_bf16_kernel (the reference rounds probabilities after the full-row

@@ -156,8 +156,11 @@ def _decode_mode(num_splits: int, pairs: int, layer: LayerKVCache) -> int:
     for bf16 rows of at most 512 slots at head dim 256 over so few (b, kv head) pairs that a row on two
     CUs is the longer chain, or over more pairs than the one-launch kernel's two workgroups per pair
     have CUs (us per call, one / two launches: 2 pairs 10.7 / 9.3, 32 pairs 11.5 / 10.6, 64 pairs
-    11.9 / 12.3, 128 pairs 15.9 / 17.1, 192 pairs 26.8 / 24.2; at head dim 128 one launch is as fast
-    or faster at every count). The library's own choice there is the path without a workspace."""
+    11.9 / 12.3, 128 pairs 15.9 / 17.1, 192 pairs 26.8 / 24.2; a full 512-slot ring at R = 1 / 16: 1 pair
+    10.2 / 8.7, 13.8 / 11.7, 32 pairs 11.4 / 10.6, 14.7 / 13.0, 160 pairs 23.1 / 21.0, 29.9 / 25.3, 224 pairs
+    28.6 / 24.3, 34.4 / 28.8, 255 pairs 29.5 / 29.8, 35.7 / 34.7; 128 slots, R = 4: 160 pairs 18.6 / 12.0; at
+    head dim 128 one launch is as fast or faster at every count). The library's own choice there is the path
+    without a workspace."""
 
     if (num_splits == 0 and layer.key.dtype == torch.bfloat16 and layer.head_dim == 256 and layer.capacity <= 512
             and (pairs <= 32 or 128 < pairs < 256)):

@@ -6,8 +6,10 @@ torch device tensors. On first use each params object is packed once into the ke
 layout (``PackedWeights``): q/k/v projections fused into one ``[M, (H*R + 2H)*D]`` matrix with
 query columns in (kv head, r) order, o_proj rows in the same order, gate|up fused; the MLP
 matrices are stored output-major (``[N, K]``), which hipBLASLt runs faster at decode batch sizes. Per layer the
-forward runs one hipBLASLt GEMM for q/k/v, the native ``g4_kv_append`` (q/k norms, RoPE, v norm,
-cache append), the native prefill or decode attention kernel, and GEMMs for o_proj and the MLP.
+forward runs one GEMM for q/k/v, the native ``g4_kv_append`` (q/k norms, RoPE, v norm, cache append; in a
+graphed step's two-launch attention, part of it), the native prefill or decode attention kernel, and GEMMs for
+o_proj and the MLP: hipBLASLt's, native for a decode batch (gate/up and down up to 256 rows, q/k/v and o up to
+192, ``_native_proj``).
 The norm / residual / activation glue runs as three fused native kernels per layer with the
 reference's f32 rounding points: ``g4_residual_norm`` (post-attention norm + residual + pre-MLP
 norm, and post-MLP norm + residual + layer scalar + the next layer's input norm) and
