@@ -293,13 +293,13 @@ def _native_proj(x: torch.Tensor, w_t: torch.Tensor) -> bool:
     """Whether a projection runs as g4_linear_bf16: a bf16 decode batch of at most 192 rows (64 from 4096
     columns), shapes where its few-row kernel is the faster one, and both operands as it loads them (16-byte
     aligned; an embedding may be a view at any offset), no derivative following them (the library's product
-    has one: logits of a vocabulary that the LM-head kernel does not take). At 256 rows the library's tiles fill (q/k/v 13.0 / 12.0
-    us, o 11.6 / 8.8) and it stays: 132 us, 3 % of that step, for outputs that round from another f32 order."""
+    has one: logits of a vocabulary that the LM-head kernel does not take). At 256 rows the library stays (E2B
+    q/k/v 13.0 / 12.0 us, o 11.6 / 8.8: 132 us, 3 % of that step, for outputs from another f32 order)."""
 
     (rows, k), n = x.shape, w_t.shape[0]
-    return (x.is_cuda and x.dtype == torch.bfloat16 and w_t.dtype == torch.bfloat16 and not _followed(x, w_t)
+    return (x.is_cuda and x.dtype == torch.bfloat16 and w_t.dtype == torch.bfloat16
             and 0 < rows <= (64 if n >= 4096 else 192) and k <= _native_proj_k(rows, n) and n % 64 == 0 and k % 64 == 0
-            and n * k < 2 ** 30 and x.is_contiguous() and w_t.is_contiguous()
+            and n * k < 2 ** 30 and x.is_contiguous() and w_t.is_contiguous() and not _followed(x, w_t)
             and x.data_ptr() % 16 == 0 and w_t.data_ptr() % 16 == 0)
 
 

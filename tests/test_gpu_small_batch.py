@@ -211,9 +211,10 @@ def test_lm_head_fallback_keeps_its_derivatives(device):
     with torch.no_grad():
         assert M._native_proj(x[:, 0].contiguous(), e)
     for operand in (x, e):
-        leaf = operand.clone().requires_grad_()
-        logits = M.forward_lm_head(leaf if operand is e else e, leaf if operand is x else x, None)
-        (grad,) = torch.autograd.grad(logits.float().sum(), leaf)
+        with torch.enable_grad():  # other tests turn gradients off for the process
+            leaf = operand.clone().requires_grad_()
+            logits = M.forward_lm_head(leaf if operand is e else e, leaf if operand is x else x, None)
+            (grad,) = torch.autograd.grad(logits.float().sum(), leaf)
         ref = e.float().sum(0).expand(4, 1, 64) if operand is x else x.float().sum((0, 1)).expand(192, 64)
         assert torch.allclose(grad.float(), ref, rtol=2.0 ** -7, atol=2.0 ** -4)
     tangent = torch.ones_like(x)
